@@ -417,9 +417,10 @@ struct ElemArgs {
 };
 
 // Occupancy target (waves per SIMD; 4 = at most 128 VGPRs) of the default
-// instances: the FP32 laws written in closed form are held to 4; the Prony
-// laws (5, 7), Ogden's eigen-decomposition (6), the fibre law (8) and the
-// FP64 instances are not held.  WAVES > 0 overrides it (the FP32 run-loop
+// instances: the FP32 laws written in closed form are held to 4 and the FP64
+// laws without Prony history to 2 (256 VGPRs; a few registers over would
+// leave one wave); the FP32 Prony laws (5, 7), Ogden's law (6), the fibre law
+// (8) and the FP64 Prony laws are not held.  WAVES > 0 overrides it (the FP32 run-loop
 // instances are compiled for WAVES = 1..5 and the tuner picks one per
 // material segment).
 #ifndef FT_ELEM_WAVES_FP32
@@ -427,7 +428,9 @@ struct ElemArgs {
 #endif
 template <typename R, int MAT, int WAVES>
 constexpr int elem_waves() {
-  return WAVES > 0 ? WAVES : ((sizeof(R) == 4 && MAT <= 4 && MAT != -1) ? FT_ELEM_WAVES_FP32 : 1);
+  if (WAVES > 0) return WAVES;
+  if (sizeof(R) == 4) return MAT <= 4 && MAT != -1 ? FT_ELEM_WAVES_FP32 : 1;
+  return MAT > 0 && MAT != 5 && MAT != 7 ? 2 : 1;
 }
 constexpr int kMaxTuneWaves = 5;
 
