@@ -56,3 +56,15 @@ def check(km, mat, fp32, strain, angle, alpha=-4.4, seed=0):
 def test_forms_over_strain_and_rotation(km, mat, fp32, strain, angle):  # noqa: F811
     check(km, mat, fp32, strain, angle)
 
+
+@pytest.mark.parametrize("fp32", [0, 1])
+@pytest.mark.parametrize("alpha", [2.0, 4.0, -2.0, 20.0, -20.0, 0.5])
+@pytest.mark.parametrize("strain", [1e-4, 0.03, 0.12, 0.4, 0.8])
+def test_ogden_exponents(km, request, fp32, alpha, strain):  # noqa: F811
+    """Exponents whose series ends (positive even), converges slowly or is
+    left for the principal directions."""
+    if fp32 and alpha == -20.0 and strain == 0.8:
+        # the stretches' FP32 round-off comes out multiplied by |alpha|, which the bound leaves out: 3.9e-6 here
+        # with the principal directions alone too, against 2.1e-6
+        request.applymarker(pytest.mark.xfail(strict=True, reason="condition |alpha| of the FP32 stretches"))
+    check(km, 7, fp32, strain, 0.1, alpha, seed=3)
