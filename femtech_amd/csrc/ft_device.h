@@ -514,35 +514,28 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
     // LinearElastic.cpp:14-70: P = lambda tr(eps) I + 2 mu eps, S = F^-1 P,
     // unsymmetrised, upper triangle kept.
     R trE = H[0][0] + H[1][1] + H[2][2];
+    // (the fused products are written out: left to the compiler, their choice
+    // differed between the kernels that share this routine)
     R P[3][3];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j) P[i][j] = mu * (H[i][j] + H[j][i]);
-    P[0][0] += lambda * trE;
-    P[1][1] += lambda * trE;
-    P[2][2] += lambda * trE;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) P[i][i] = Num<R>::fma_(lambda, trE, mu * (H[i][i] + H[i][i]));
     R F[3][3];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j) F[i][j] = H[i][j] + (i == j ? R(1) : R(0));
     R A[3][3];  // adj(F)
-    A[0][0] = F[1][1] * F[2][2] - F[1][2] * F[2][1];
-    A[0][1] = F[0][2] * F[2][1] - F[0][1] * F[2][2];
-    A[0][2] = F[0][1] * F[1][2] - F[0][2] * F[1][1];
-    A[1][0] = F[1][2] * F[2][0] - F[1][0] * F[2][2];
-    A[1][1] = F[0][0] * F[2][2] - F[0][2] * F[2][0];
-    A[1][2] = F[0][2] * F[1][0] - F[0][0] * F[1][2];
-    A[2][0] = F[1][0] * F[2][1] - F[1][1] * F[2][0];
-    A[2][1] = F[0][1] * F[2][0] - F[0][0] * F[2][1];
-    A[2][2] = F[0][0] * F[1][1] - F[0][1] * F[1][0];
+    adjugate(F, A);
     R iJ = Num<R>::rcp_(R(1) + Jm1);
     const int I[6] = {0, 1, 2, 1, 0, 0}, J[6] = {0, 1, 2, 2, 2, 1};
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
       int i = I[k], j = J[k];
-      S.v[k] = (A[i][0] * P[0][j] + A[i][1] * P[1][j] + A[i][2] * P[2][j]) * iJ;
+      S.v[k] = Num<R>::fma_(A[i][2], P[2][j], Num<R>::fma_(A[i][1], P[1][j], A[i][0] * P[0][j])) * iJ;
     }
     return true;
   }
@@ -1253,6 +1246,91 @@ constexpr int kFlagNonFinite = 1;
 constexpr int kFlagInverted = 2;
 constexpr int kFlagMaterial = 8;
 
+// Per-Gauss-point fields of FemTech's element layer for one element, in the
+// reference's layout (ShapeFunctions.cpp:174-205 with 8 Gauss points): F
+// (9 per point, column-major), det F (1) and the PK2 stress (6, Voigt).
+struct GpSink {
+  double *F, *detF, *pk2;
+};
+
+// Prony coefficients of a step (HGOIsotropicViscoelastic.cpp:126-131, global
+// dt); zero for the laws without history.
+__host__ __device__ inline ViscoCoef visco_coef(int mat, const PartDev &pp, double dt_step) {
+  ViscoCoef vc = {0, 0, 0, 0};
+  if (mat == 5 || mat == 7) {
+    const double rt1 = dt_step / pp.t1, rt2 = dt_step / pp.t2;
+    vc.c11 = exp(-rt1);
+    vc.c12 = exp(-rt2);
+    vc.c21 = pp.g1 * (1 - vc.c11) / rt1;
+    vc.c22 = pp.g2 * (1 - vc.c12) / rt2;
+  }
+  return vc;
+}
+
+// One Gauss point: Q = w det(J0) P J0^-T (w = 1) from the Jacobians J0 =
+// d(X)/d(xi) and Ju = d(u)/d(xi) (each 8 x, so Q is 64 x), so that f_a,i =
+// sum_gp sum_k Q_ik dN_a/dxi_k.  `hist` as for element_eval; gps receives
+// the point's fields with GPOUT.
+template <typename R, int MAT, class Hist, bool SURR, bool GPOUT>
+__host__ __device__ inline void gauss_point_q(const R J0[3][3], const R Ju[3][3], const PartDev &pp, const R fib[3],
+                                              int gp, Hist &hist, bool update_hist, const ViscoCoef &vc, R Q[3][3],
+                                              int &flags, const SurrIn *sin, SurrTally *tally, const GpSink *gps) {
+  const int mat = MAT >= 0 ? MAT : pp.mat;
+  // adj(J0): J0^-1 = A / det0 (ShapeFunction_C3D8.cpp:95-123)
+  R A[3][3];
+  adjugate(J0, A);
+  const R det0 = J0[0][0] * A[0][0] + J0[0][1] * A[1][0] + J0[0][2] * A[2][0];
+  if (!(det0 > R(0))) flags |= kFlagInverted;
+  const R idet0 = Num<R>::rcp_(det0);
+  // H = Ju J0^-1 = grad_X u  (F = I + H, CalculateDeformationGradient.cpp:15-25)
+  R H[3][3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      H[i][j] = (Ju[i][0] * A[0][j] + Ju[i][1] * A[1][j] + Ju[i][2] * A[2][j]) * idet0;
+  R P[3][3], Jm1;  // P = F S (first Piola)
+  if constexpr ((MAT == 1 || MAT == 4 || MAT == 8) && !SURR && !GPOUT) {
+    first_piola<R, MAT>(pp, H, fib, P, Jm1);
+    if (!(Jm1 > R(-1))) flags |= kFlagInverted;
+  } else {
+    // history of this Gauss point, in registers (fixed-size array, static
+    // indices: no private-memory copy)
+    R hloc[18];
+    const bool use_hist = (mat == 5 || mat == 7) && hist.valid();
+#pragma unroll
+    for (int k = 0; k < 18; ++k) hloc[k] = use_hist ? hist.load(gp, k) : R(0);
+    Sym<R> S;
+    if constexpr (SURR) {
+      surr_pk2<R, MAT>(pp, H, fib, *sin, gp, hloc, use_hist, vc, S, Jm1, *tally);
+    } else {
+      if (!pk2_stress<R, MAT>(pp, H, hloc, use_hist, vc, S, Jm1)) flags |= kFlagMaterial;
+    }
+    if (!(Jm1 > R(-1))) flags |= kFlagInverted;
+    if (use_hist && update_hist) {
+#pragma unroll
+      for (int k = 0; k < 18; ++k) hist.store(gp, k, hloc[k]);
+    }
+    if constexpr (GPOUT) {
+      // F = I + H (CalculateDeformationGradient.cpp:14 layout), det F, S
+      for (int i = 0; i < 3; ++i)
+        for (int j = 0; j < 3; ++j) gps->F[9 * gp + 3 * j + i] = (double)H[i][j] + (i == j ? 1.0 : 0.0);
+      gps->detF[gp] = 1.0 + (double)Jm1;
+      for (int k = 0; k < 6; ++k) gps->pk2[6 * gp + k] = (double)S.v[k];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        P[i][j] = sym_at(S, i, j) + H[i][0] * sym_at(S, 0, j) + H[i][1] * sym_at(S, 1, j) +
+                  H[i][2] * sym_at(S, 2, j);
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) Q[i][k] = P[i][0] * A[k][0] + P[i][1] * A[k][1] + P[i][2] * A[k][2];
+}
+
 // One element from the unnormalised Walsh-Hadamard coefficients of its
 // reference coordinates (cx) and displacements (cu): c[m][d] = sum_p
 // sign_m(p) v_d(p) over the 8 nodes in cube-position order p (see p2n), m =
@@ -1265,13 +1343,6 @@ constexpr int kFlagMaterial = 8;
 // order (node-major, xyz) and lowers dt_e when DT is set and the element is
 // not skipped.  `hist` is an accessor with load(gp, k) / store(gp, k, v) for
 // the 18 Prony values of a Gauss point (materials 5 and 7).
-// Per-Gauss-point fields of FemTech's element layer for one element, in the
-// reference's layout (ShapeFunctions.cpp:174-205 with 8 Gauss points): F
-// (9 per point, column-major), det F (1) and the PK2 stress (6, Voigt).
-struct GpSink {
-  double *F, *detF, *pk2;
-};
-
 template <typename R, bool FORCE, bool DT, int MAT, class Hist, bool SURR = false, bool GPOUT = false>
 __host__ __device__ inline void element_eval(R cx[7][3], R cu[7][3], const PartDev &pp,
                                              bool skip_dt, double dt_step, Hist &hist,
@@ -1306,14 +1377,7 @@ __host__ __device__ inline void element_eval(R cx[7][3], R cu[7][3], const PartD
 #pragma unroll
     for (int k = 0; k < 24; ++k) outv[k] = R(0);
   } else if (FORCE) {
-    ViscoCoef vc = {0, 0, 0, 0};
-    if (mat == 5 || mat == 7) {  // HGOIsotropicViscoelastic.cpp:126-131, global dt
-      const double rt1 = dt_step / pp.t1, rt2 = dt_step / pp.t2;
-      vc.c11 = exp(-rt1);
-      vc.c12 = exp(-rt2);
-      vc.c21 = pp.g1 * (1 - vc.c11) / rt1;
-      vc.c22 = pp.g2 * (1 - vc.c12) / rt2;
-    }
+    const ViscoCoef vc = visco_coef(mat, pp, dt_step);
     const R g = R(kGp), g2 = R(kGp * kGp);
     R h[3][7];  // force accumulators in the monomial basis
 #pragma unroll
@@ -1372,74 +1436,10 @@ __host__ __device__ inline void element_eval(R cx[7][3], R cu[7][3], const PartD
         Ju[d][1] = Num<R>::fma_(sx, cu[2][d], cu[1][d]);
         Ju[d][2] = Num<R>::fma_(gxy, cu[6][d], Num<R>::fma_(gy, cu[5][d], Num<R>::fma_(gx, cu[4][d], cu[3][d])));
       }
-      // adj(J0): J0^-1 = A / det0 (ShapeFunction_C3D8.cpp:95-123)
-      R A[3][3];
-      adjugate(J0, A);
-      const R det0 = J0[0][0] * A[0][0] + J0[0][1] * A[1][0] + J0[0][2] * A[2][0];
-      if (!(det0 > R(0))) flags |= kFlagInverted;
-      const R idet0 = Num<R>::rcp_(det0);
-      // H = Ju J0^-1 = grad_X u  (F = I + H, CalculateDeformationGradient.cpp:15-25)
-      R H[3][3];
+      R Q[3][3];
+      gauss_point_q<R, MAT, Hist, SURR, GPOUT>(J0, Ju, pp, fib, gp, hist, update_hist, vc, Q, flags, sin, tally, gps);
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          H[i][j] = (Ju[i][0] * A[0][j] + Ju[i][1] * A[1][j] + Ju[i][2] * A[2][j]) * idet0;
-      if constexpr ((MAT == 1 || MAT == 4 || MAT == 8) && !SURR && !GPOUT) {
-        R P[3][3];
-        R Jm1;
-        first_piola<R, MAT>(pp, H, fib, P, Jm1);
-        if (!(Jm1 > R(-1))) flags |= kFlagInverted;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          const R q0 = P[i][0] * A[0][0] + P[i][1] * A[0][1] + P[i][2] * A[0][2];
-          const R q1 = P[i][0] * A[1][0] + P[i][1] * A[1][1] + P[i][2] * A[1][2];
-          const R q2 = P[i][0] * A[2][0] + P[i][1] * A[2][1] + P[i][2] * A[2][2];
-          accumulate_force_basis(h[i], q0, q1, q2, gw);
-        }
-        continue;
-      }
-      // history of this Gauss point, in registers (fixed-size array, static
-      // indices: no private-memory copy)
-      R hloc[18];
-      const bool use_hist = (mat == 5 || mat == 7) && hist.valid();
-#pragma unroll
-      for (int k = 0; k < 18; ++k) hloc[k] = use_hist ? hist.load(gp, k) : R(0);
-      Sym<R> S;
-      R Jm1;
-      if constexpr (SURR) {
-        surr_pk2<R, MAT>(pp, H, fib, *sin, gp, hloc, use_hist, vc, S, Jm1, *tally);
-      } else {
-        if (!pk2_stress<R, MAT>(pp, H, hloc, use_hist, vc, S, Jm1)) flags |= kFlagMaterial;
-      }
-      if (!(Jm1 > R(-1))) flags |= kFlagInverted;
-      if (use_hist && update_hist) {
-#pragma unroll
-        for (int k = 0; k < 18; ++k) hist.store(gp, k, hloc[k]);
-      }
-      if constexpr (GPOUT) {
-        // F = I + H (CalculateDeformationGradient.cpp:14 layout), det F, S
-        for (int i = 0; i < 3; ++i)
-          for (int j = 0; j < 3; ++j) gps->F[9 * gp + 3 * j + i] = (double)H[i][j] + (i == j ? 1.0 : 0.0);
-        gps->detF[gp] = 1.0 + (double)Jm1;
-        for (int k = 0; k < 6; ++k) gps->pk2[6 * gp + k] = (double)S.v[k];
-      }
-      // P = F S (first Piola), Q = w detJ0 P J0^-T = P A^T  (w = 1)
-      R P[3][3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          P[i][j] = sym_at(S, i, j) + H[i][0] * sym_at(S, 0, j) + H[i][1] * sym_at(S, 1, j) +
-                    H[i][2] * sym_at(S, 2, j);
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const R q0 = P[i][0] * A[0][0] + P[i][1] * A[0][1] + P[i][2] * A[0][2];
-        const R q1 = P[i][0] * A[1][0] + P[i][1] * A[1][1] + P[i][2] * A[1][2];
-        const R q2 = P[i][0] * A[2][0] + P[i][1] * A[2][1] + P[i][2] * A[2][2];
-        // f_a,i = sum_gp sum_k Q_ik dN_a/dxi_k in the monomial basis
-        accumulate_force_basis(h[i], q0, q1, q2, gw);
-      }
+      for (int i = 0; i < 3; ++i) accumulate_force_basis(h[i], Q[i][0], Q[i][1], Q[i][2], gw);
     }
     // Back to the nodes: f_p = sum_q c_q prod(signs) (h carries the scale).
 #pragma unroll

@@ -89,6 +89,7 @@ constexpr int kExtraFree = 20;
 // (its first wavefront's shadow lane computes it)
 constexpr int kTileShadows = 4;
 constexpr int kTileShadow = 2;
+constexpr int kTileMat = 8;  // material id of an element tile: flags >> kTileMat
 constexpr int kPidMask = (1 << 20) - 1;
 constexpr int kMaxMotions = 64;  // distinct motions per instance (held in LDS by the nodal kernel)
 constexpr int kEaccStride = 8;  // doubles per nodal block in the energy accumulators
@@ -700,6 +701,337 @@ __device__ __forceinline__ void element_tile(const ElemArgs<R> &a, const int L) 
 template <typename R, bool FORCE, bool DT, int MAT, int WAVES>
 __global__ __launch_bounds__(kBlock, (elem_waves<R, MAT, WAVES>())) void k_element(ElemArgs<R> a) {
   element_tile<R, FORCE, DT, MAT>(a, xcd_block());
+}
+
+// ---------------------------------------------------------------------------
+// FP64 element kernel of small segments: a block of 8 wavefronts per 64 elements,
+// one Gauss point per wavefront.
+// ---------------------------------------------------------------------------
+// k_element evaluates an element's 8 Gauss points one after another in one
+// lane: about 3,500 dependent instructions, however few elements there are.
+// Here lane l of all 8 wavefronts belongs to the same element; wavefront w
+// (wave-uniform signs, coalesced Prony history) takes Gauss point w, and the
+// wavefronts exchange through LDS:
+//   1. wavefronts 0-5: one component of X or u each: gather 8 nodes, Walsh-
+//      Hadamard transform (FP64), and the 12 distinct Jacobian entries of that
+//      component over the 8 points; those of u also transform X + u for the
+//      time step;
+//   2. all: wavefront w's six face areas / volume of the time step (w < 7),
+//      then Gauss point w (gauss_point_q);
+//   3. the 21 force coefficients in the monomial basis, shared out over the
+//      wavefronts, each summed over the points in order;
+//   4. all: the force of node w from them, corner pairs through LDS.
+// Every sum keeps element_eval's operations and order, so which kernel a
+// segment takes shows in a run by no more than the compiler's own choice of
+// fused products.  A block covers the elements of one wavefront of the
+// segment's tiles (63 behind a shadow lane with corner pairs, else 64), so
+// both kernels pair alike and keep the same slots.  FP64 only: the FP32 run
+// loop refines the step size of one element per tile, and a minimum over
+// other groups of elements would differ from it in the last bits.
+// Up to some 10,000 elements the launch is a chain of memory round trips, four
+// barriers and one Gauss point (FP64 neo-Hookean, 1,000 elements: 14.7 -> 8.6
+// us).  The arithmetic is twice k_element's and more, so the kernel is for
+// segments that leave the chip's wavefront slots idle otherwise (wave_cost).
+constexpr int kWaveBlock = 512;
+
+struct WaveLds {
+  using R = double;
+  union {
+    R J[6][12][64];   // Jacobian entries: X then u by component; 4 each of d/dxi, d/deta, d/dzeta
+    R Q[72][64];      // Q of Gauss point gp: rows 9 gp + 3 i + k
+    R pair[4][3][64]; // xi+ corner forces for the right lane
+  };
+  union {
+    double C[3][7][64];  // Walsh-Hadamard coefficients of X + u (time step)
+    R h[21][64];         // force coefficients: rows 7 i + m (element_eval's h)
+  };
+  double part[7][64];  // face areas and volume
+};
+
+// Force coefficient m of component i (element_eval's h[i][m]): the columns of
+// Q it takes and the coordinates whose signs weigh them
+// (accumulate_force_basis), summed over the Gauss points in order.
+template <int M>
+__device__ __forceinline__ double wave_force_coef(const double (&Q)[72][64], int i, int lane) {
+  using R = double;
+  constexpr int terms = (M == 0 || M == 1 || M == 3) ? 1 : (M == 6 ? 3 : 2);
+  // columns; coordinate masks (1: xi, 2: eta, 4: zeta)
+  constexpr int col[7][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {2, 0, 0}, {0, 2, 0}, {1, 2, 0}, {0, 1, 2}};
+  constexpr int msk[7][3] = {{0, 0, 0}, {0, 0, 0}, {2, 1, 0}, {0, 0, 0}, {4, 1, 0}, {4, 2, 0}, {6, 5, 3}};
+  const R g = R(kGp), g2 = R(kGp * kGp);
+  const R wt = terms == 1 ? R(0.125 / 64) : terms == 2 ? g * R(0.125 / 64) : g2 * R(0.125 / 64);
+  R acc = R(0);
+#pragma unroll
+  for (int gp = 0; gp < 8; ++gp) {
+    const unsigned neg = (((gp ^ (gp >> 1)) & 1) ^ 1) | ((((gp >> 1) & 1) ^ 1) << 1) | (((gp >> 2) & 1) << 2);
+#pragma unroll
+    for (int t = 0; t < terms; ++t) {
+      const unsigned b = neg & (unsigned)msk[M][t];
+      acc = Num<R>::fma_(flip_sign(wt, (b ^ (b >> 1) ^ (b >> 2)) & 1u), Q[9 * gp + 3 * i + col[M][t]][lane], acc);
+    }
+  }
+  return acc;
+}
+
+// The laws a merged launch dispatches on (kAllLaws), or a single one.
+constexpr int kAllLaws = -1;
+template <int MAT>
+__device__ inline void wave_gauss_point(int mat, const double J0[3][3], const double Ju[3][3], const PartDev &pp,
+                                        const double fib[3], int gp, HistSoA<double> &hist, bool update,
+                                        const ViscoCoef &vc, double Q[3][3], int &flags) {
+  using R = double;
+  if constexpr (MAT != kAllLaws) {
+    gauss_point_q<R, MAT, HistSoA<R>, false, false>(J0, Ju, pp, fib, gp, hist, update, vc, Q, flags, nullptr, nullptr,
+                                                    nullptr);
+  } else {
+    switch (mat) {  // uniform over the block
+      case 1: return wave_gauss_point<1>(mat, J0, Ju, pp, fib, gp, hist, update, vc, Q, flags);
+      case 2: return wave_gauss_point<2>(mat, J0, Ju, pp, fib, gp, hist, update, vc, Q, flags);
+      case 3: return wave_gauss_point<3>(mat, J0, Ju, pp, fib, gp, hist, update, vc, Q, flags);
+      case 4: return wave_gauss_point<4>(mat, J0, Ju, pp, fib, gp, hist, update, vc, Q, flags);
+      case 5: return wave_gauss_point<5>(mat, J0, Ju, pp, fib, gp, hist, update, vc, Q, flags);
+      case 6: return wave_gauss_point<6>(mat, J0, Ju, pp, fib, gp, hist, update, vc, Q, flags);
+      case 7: return wave_gauss_point<7>(mat, J0, Ju, pp, fib, gp, hist, update, vc, Q, flags);
+      case 8: return wave_gauss_point<8>(mat, J0, Ju, pp, fib, gp, hist, update, vc, Q, flags);
+    }
+  }
+}
+
+template <int MAT>
+__global__ __launch_bounds__(kWaveBlock) void k_element_waves(ElemArgs<double> a, int per_tile) {
+  using R = double;
+  __shared__ WaveLds lds;
+  const int L = xcd_block();
+  const int ti = L / per_tile, sub = L - ti * per_tile;
+  if (ti >= a.n_tiles) return;  // grid padding (uniform over the block, as every return here)
+  const int4 tile = a.tiles[ti];
+  const int end = tile.y;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // element of this lane: the same as lane `lane` of wavefront `sub` of the tile in k_element
+  int e = tile.x + 64 * sub + lane;
+  bool owner = true, active = e < end;
+  if (a.pair && (tile.w & kTileShadows)) {
+    e = tile.x + 63 * sub + lane - 1;
+    if (e + 1 - lane >= end) return;
+    owner = lane != 0;
+    active = owner ? e < end : (sub != 0 || (tile.w & kTileShadow));
+  } else if (e - lane >= end) {
+    return;
+  }
+  double dt_step = a.dt_fixed;
+  unsigned long long *dtmin = a.dtbits ? a.dtbits + tile.z : nullptr;
+  if (a.ctl) {
+    const StepSlot *slot = &a.ctl[tile.z].slot[a.parity];
+    if (slot->done) return;
+    dt_step = slot->dt;
+    dtmin = &a.ctl[tile.z].slot[a.parity].dtmin_bits;
+  }
+  const int mat = tile.w >> kTileMat;
+  const bool force = a.want_force && mat != 0;
+  int node = 0, info = 0;
+  PartDev pp;
+  if (active) {
+    info = a.einfo[e];
+    const int4 *c4 = reinterpret_cast<const int4 *>(a.conn) + 2 * (size_t)e;
+    if (w < 6) {
+      const int4 c0 = c4[0], c1 = c4[1];
+      const int nd[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+      const double *src = w < 3 ? a.X + (size_t)w * a.nn : a.u + (size_t)(w - 3) * a.nn;
+      double v[8], y[8];
+#pragma unroll
+      for (int p = 0; p < 8; ++p) v[p] = src[nd[p2n(p)]];
+      if (a.want_dt && w >= 3) {
+        const double *Xc = a.X + (size_t)(w - 3) * a.nn;
+#pragma unroll
+        for (int p = 0; p < 8; ++p) y[p] = Xc[nd[p2n(p)]];
+        wht8(y);
+      }
+      wht8(v);
+      if (a.want_dt && w >= 3)
+#pragma unroll
+        for (int m = 0; m < 7; ++m)
+          lds.C[w - 3][m][lane] = 0.125 * (y[m + 1] + v[m + 1]);
+      if (force) {
+        R c[7];
+#pragma unroll
+        for (int m = 0; m < 7; ++m) c[m] = R(v[m + 1]);
+        // element_eval's Jacobian columns on the planes zeta = +, - (bits of an index, set: +)
+        const R g = R(kGp), g2 = R(kGp * kGp);
+        R a0 = Num<R>::fma_(g, c[4], c[0]), a1 = Num<R>::fma_(g, c[5], c[1]), b0 = Num<R>::fma_(g2, c[6], g * c[2]);
+#pragma unroll
+        for (int z = 1; z >= 0; --z) {
+          lds.J[w][2 * z][lane] = a0 - b0;  // d/dxi at [sy + 2 sz]
+          lds.J[w][2 * z + 1][lane] = a0 + b0;
+          lds.J[w][4 + 2 * z][lane] = a1 - b0;  // d/deta at [sx + 2 sz]
+          lds.J[w][4 + 2 * z + 1][lane] = a1 + b0;
+          a0 = Num<R>::fma_(R(-2) * g, c[4], a0);
+          a1 = Num<R>::fma_(R(-2) * g, c[5], a1);
+          b0 = Num<R>::fma_(R(-2) * g2, c[6], b0);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {  // d/dzeta at [sx + 2 sy]
+          const R gx = (q & 1) ? g : -g, gy = (q & 2) ? g : -g, gxy = q == 0 || q == 3 ? g2 : -g2;
+          lds.J[w][8 + q][lane] =
+              Num<R>::fma_(gxy, c[6], Num<R>::fma_(gy, c[5], Num<R>::fma_(gx, c[4], c[3])));
+        }
+      }
+    }
+    node = a.conn[8 * (size_t)e + p2n(w)];
+    pp = a.parts[info & kPidMask];
+  }
+  __syncthreads();
+  if (a.want_dt && w < 7 && active) {
+    // face areas in the order of CalculateCharacteristicLength_C3D8.cpp:12-13
+    // and the volume, as hex_part, from the coefficients each of them needs
+    auto c3 = [&](int m, double v[3]) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) v[k] = lds.C[k][m][lane];
+    };
+    if (w == 6) {
+      double d[7][3];
+#pragma unroll
+      for (int m = 0; m < 6; ++m) c3(m, d[m]);
+      lds.part[6][lane] = hex_part(d, 6);
+    } else {
+      // (twist, edge, edge) of the face pair: one coefficient +- another
+      const int g = w >> 1;
+      const int m0[3] = {g == 0 ? 2 : g == 1 ? 5 : 4, g == 1 ? 1 : 0, g == 0 ? 1 : 3};
+      const int m1[3] = {6, g == 0 ? 4 : 2, g == 1 ? 4 : 5};
+      const double sg = (w & 1) ? 1.0 : -1.0;
+      double f[3][3], h[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        c3(m0[j], f[j]);
+        c3(m1[j], h);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) f[j][k] += sg * h[k];
+      }
+      lds.part[w][lane] = face_area(f[0], f[1], f[2]);
+    }
+  }
+  R Q[3][3];
+  int flags = 0;
+  if (force && active) {
+    // Gauss point w (GaussQuadrature3D.cpp:19-49)
+    const int sx = (w ^ (w >> 1)) & 1, sy = (w >> 1) & 1, sz = (w >> 2) ^ 1;
+    R J0[3][3], Ju[3][3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      J0[d][0] = lds.J[d][sy + 2 * sz][lane];
+      J0[d][1] = lds.J[d][4 + sx + 2 * sz][lane];
+      J0[d][2] = lds.J[d][8 + sx + 2 * sy][lane];
+      Ju[d][0] = lds.J[3 + d][sy + 2 * sz][lane];
+      Ju[d][1] = lds.J[3 + d][4 + sx + 2 * sz][lane];
+      Ju[d][2] = lds.J[3 + d][8 + sx + 2 * sy][lane];
+    }
+    R fib[3] = {R(1), R(0), R(0)};
+    if (mat == 8 && a.fib) {
+      fib[0] = a.fib[e];
+      fib[1] = a.fib[(size_t)a.ne + e];
+      fib[2] = a.fib[2 * (size_t)a.ne + e];
+    }
+    HistSoA<R> hist{a.hist, a.ne, e};
+    const ViscoCoef vc = visco_coef(mat, pp, dt_step);
+    wave_gauss_point<MAT>(mat, J0, Ju, pp, fib, w, hist, a.update_hist != 0 && owner, vc, Q, flags);
+  }
+  __syncthreads();
+  if (a.want_dt && w == 7) {
+    // StableTimeStep.cpp:11-30: Le / ce on the deformed geometry (FP64)
+    double dte = 1e300;
+    if (active && !(info & kSkipBit)) {
+      double amax = 0.0;
+      for (int f = 0; f < 6; ++f) amax = lds.part[f][lane] > amax ? lds.part[f][lane] : amax;
+      const double d = lds.part[6][lane] / amax / pp.ce;
+      if (d < dte) dte = d;  // NaN never lowers the minimum
+    }
+    for (int o = 32; o > 0; o >>= 1) dte = fmin(dte, __shfl_xor(dte, o));
+    if (lane == 0 && dte < 1e300 && dtmin) atomicMin(dtmin, dt_key(dte));
+  }
+  if (!a.want_force) {
+    if (flags) atomicOr(a.status, flags);
+    return;
+  }
+  if (force) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) lds.Q[9 * w + 3 * i + k][lane] = Q[i][k];
+  }
+  __syncthreads();
+  if (force) {
+    // at most 40 of the 288 products of a coefficient each
+    switch (w) {
+#define FT_WAVE_COEF(i, m) lds.h[7 * (i) + (m)][lane] = wave_force_coef<m>(lds.Q, i, lane)
+      case 0: FT_WAVE_COEF(0, 6); FT_WAVE_COEF(0, 0); break;
+      case 1: FT_WAVE_COEF(1, 6); FT_WAVE_COEF(1, 0); break;
+      case 2: FT_WAVE_COEF(2, 6); FT_WAVE_COEF(2, 0); break;
+      case 3: FT_WAVE_COEF(0, 2); FT_WAVE_COEF(1, 2); FT_WAVE_COEF(0, 1); break;
+      case 4: FT_WAVE_COEF(2, 2); FT_WAVE_COEF(0, 4); FT_WAVE_COEF(1, 1); break;
+      case 5: FT_WAVE_COEF(1, 4); FT_WAVE_COEF(2, 4); FT_WAVE_COEF(2, 1); break;
+      case 6: FT_WAVE_COEF(0, 5); FT_WAVE_COEF(1, 5); FT_WAVE_COEF(0, 3); break;
+      case 7: FT_WAVE_COEF(2, 5); FT_WAVE_COEF(1, 3); FT_WAVE_COEF(2, 3); break;
+#undef FT_WAVE_COEF
+    }
+  }
+  __syncthreads();
+  R f[3] = {R(0), R(0), R(0)};
+  if (force) {
+    // the node at cube position w: its branch of iwht8's tree
+    const R s0 = (w & 1) ? R(1) : R(-1), s1 = (w & 2) ? R(1) : R(-1), s2 = (w & 4) ? R(1) : R(-1);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      R c[8];
+      c[0] = R(0);
+#pragma unroll
+      for (int m = 0; m < 7; ++m) c[m + 1] = lds.h[7 * i + m][lane];
+      const R x0 = Num<R>::fma_(s0, c[1], c[0]), x1 = Num<R>::fma_(s0, c[3], c[2]);
+      const R x2 = Num<R>::fma_(s0, c[5], c[4]), x3 = Num<R>::fma_(s0, c[7], c[6]);
+      f[i] = Num<R>::fma_(s2, Num<R>::fma_(s1, x3, x2), Num<R>::fma_(s1, x1, x0));
+    }
+    if (!a.ctl && active && !(isfinite(f[0]) && isfinite(f[1]) && isfinite(f[2]))) flags |= kFlagNonFinite;
+  }
+  if (flags) atomicOr(a.status, flags);
+  const int k = p2n(w);
+  if (a.eslot) {  // node slots (k_element)
+    if (!active) return;
+    const unsigned r = (a.eslot[e] >> (4 * k)) & 15u;
+    R *dst = r < 8u ? a.fe + 3 * ((size_t)r * a.nn + (size_t)node)
+                    : a.fe_ovf + 3 * ((size_t)(r - 8u) * a.n_ovf + (size_t)(a.ovf[node] >> 4));
+    dst[0] = f[0];
+    dst[1] = f[1];
+    dst[2] = f[2];
+    return;
+  }
+  bool right = false, to_minus = false, extra = false;
+  if (a.pair) {  // corner pairs (k_element): wavefront w | 1 holds the left lane's xi+ corner of this face edge
+    if (w & 1)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) lds.pair[w >> 1][d][lane] = f[d];
+    __syncthreads();
+    if (!(w & 1) && (info & kPairLeft) && lane > 0)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) f[d] += lds.pair[w >> 1][d][lane - 1];
+    right = (info & kPairRight) != 0;
+    to_minus = (info & kPlusToMinus) != 0;
+    extra = (info & kExtra) != 0;
+  }
+  if (!active || !owner) return;
+  const bool plus = (w & 1) != 0;
+  if (plus && right) return;
+  if (plus && extra && !((info >> (kExtraFree + (w >> 1))) & 1)) {
+    // extras entry j of the xi+ corners 1, 2, 5, 6
+    const int j = (k >> 1 & 2) | (k == 2 || k == 6);
+    R *x = a.xf + 3 * ((size_t)a.xidx[e] + j);
+    x[0] = f[0];
+    x[1] = f[1];
+    x[2] = f[2];
+    return;
+  }
+  const int slot = plus && (to_minus || extra) ? k ^ 1 : k;
+  R *dst = a.fe + 3 * ((size_t)slot * (a.corner ? a.nn : a.ne) + (size_t)(a.corner ? node : e));
+  dst[0] = f[0];
+  dst[1] = f[1];
+  dst[2] = f[2];
 }
 
 // Forces plus FemTech's per-Gauss-point F, det F and PK2 (every law through
@@ -2525,21 +2857,95 @@ int force_segment(ft_engine *g, const ft_engine::Seg &sg, int waves, bool in_loo
   return fail(FT_ERR_MATERIAL, "Unknown material type %d", sg.mat);
 }
 
+// When k_element_waves takes a run of consecutive FP64 material segments: each
+// segment's own k_element launch costs `alone` us however small it is; as
+// part of a k_element_waves launch it costs time in proportion to its
+// elements, the same at `even` of them; and that launch itself costs
+// kWaveLaunch us.  Measured on jittered blocks of one law, us per launch of
+// k_element / k_element_waves at 1,000, 8,000, 32,768 and 97,336 elements:
+// neo-Hookean 16.8 / 11.0, 17.3 / 11.6, 18.7 / 21.3, 28.8 / 39.8; HGO + Prony
+// 27.8 / 13.4, 28.9 / 15.5, 31.4 / 29.4, 58.6 / 70.9; Ogden + Prony 83.3 /
+// 31.4, 95.0 / 29.1, 60.8 / 37.9, 90.0 / 88.5; anisotropic HGO 23.5 / 11.9,
+// 23.7 / 12.1, 25.4 / 23.3, 42.0 / 44.3.  The launch shapes of
+// ft_set_segment_shape and ft_autotune apply to k_element only.
+struct WaveCost {
+  double alone;  // us
+  int even;      // elements
+};
+constexpr double kWaveLaunch = 10.5;  // us
+WaveCost wave_cost(int mat) {
+  switch (mat) {
+    case 4: return {19, 65000};
+    case 5: return {26, 60000};
+    case 6: return {40, 120000};
+    case 7: return {60, 150000};
+    case 8: return {21, 100000};
+    default: return {15, 80000};
+  }
+}
+
+// End of the run of segments from s on that k_element_waves takes (s: none).
+size_t wave_run(const ft_engine *g, size_t s) {
+  if (g->precision == FT_FP32) return s;
+  double gain = -kWaveLaunch;
+  size_t s1 = s;
+  for (; s1 < g->segs.size(); ++s1) {
+    const WaveCost c = wave_cost(g->segs[s1].mat);
+    const int ne = g->segs[s1].end - g->segs[s1].begin;
+    if (ne >= c.even) break;
+    gain += c.alone * (1.0 - (double)ne / c.even);
+  }
+  return gain > 0.0 ? s1 : s;
+}
+
+// k_element_waves over segments [s0, s1), contiguous in the internal order.
+int launch_waves(ft_engine *g, size_t s0, size_t s1, bool force, bool dt, bool in_loop, double dt_fixed,
+                 unsigned long long *dtbits, int update_hist) {
+  ElemArgs<double> a = elem_args<double>(g, g->segs[s0].tile_begin, g->segs[s1 - 1].tile_end, in_loop, dt_fixed,
+                                         dtbits, update_hist);
+  if (a.n_tiles <= 0) return 0;
+  a.want_force = force;
+  a.want_dt = dt;
+  int per_tile = 1;
+  for (size_t s = s0; s < s1; ++s) per_tile = std::max(per_tile, g->segs[s].tile / 64);
+  const dim3 grid(grid_for_tiles((long)a.n_tiles * per_tile)), block(kWaveBlock);
+  Timed t(g, 0);
+  switch (s1 - s0 == 1 ? g->segs[s0].mat : kAllLaws) {
+    case 1: hipLaunchKernelGGL(k_element_waves<1>, grid, block, 0, g->lstream, a, per_tile); break;
+    case 2: hipLaunchKernelGGL(k_element_waves<2>, grid, block, 0, g->lstream, a, per_tile); break;
+    case 3: hipLaunchKernelGGL(k_element_waves<3>, grid, block, 0, g->lstream, a, per_tile); break;
+    case 4: hipLaunchKernelGGL(k_element_waves<4>, grid, block, 0, g->lstream, a, per_tile); break;
+    case 5: hipLaunchKernelGGL(k_element_waves<5>, grid, block, 0, g->lstream, a, per_tile); break;
+    case 6: hipLaunchKernelGGL(k_element_waves<6>, grid, block, 0, g->lstream, a, per_tile); break;
+    case 7: hipLaunchKernelGGL(k_element_waves<7>, grid, block, 0, g->lstream, a, per_tile); break;
+    case 8: hipLaunchKernelGGL(k_element_waves<8>, grid, block, 0, g->lstream, a, per_tile); break;
+    default: hipLaunchKernelGGL(k_element_waves<kAllLaws>, grid, block, 0, g->lstream, a, per_tile);
+  }
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
 template <typename R>
 int element_pass_t(ft_engine *g, bool force, bool dt, bool in_loop, double dt_fixed,
                    unsigned long long *dtbits, int update_hist) {
-  // A stand-alone stable-time-step pass always runs in FP64 (exact minimum).
-  if (!force) {
-    for (const auto &sg : g->segs) {
-      int rc = launch_element<double, false, true, -1>(g, sg.tile_begin, sg.tile_end, false, dt_fixed, dtbits, 0,
-                                                       sg.tile);
-      if (rc) return rc;
-    }
-    return 0;
-  }
-  for (const auto &sg : g->segs) {
-    int rc = dt ? force_segment<R, true>(g, sg, sg.waves, in_loop, dt_fixed, dtbits, update_hist)
+  const size_t n = g->segs.size();
+  for (size_t s = 0; s < n;) {
+    const auto &sg = g->segs[s];
+    int rc;
+    size_t s1;
+    if ((s1 = wave_run(g, s)) > s) {
+      rc = launch_waves(g, s, s1, force, dt, in_loop, dt_fixed, dtbits, update_hist);
+      s = s1;
+    } else {
+      // a stand-alone stable-time-step pass always runs in FP64 (exact minimum)
+      if (!force)
+        rc = launch_element<double, false, true, -1>(g, sg.tile_begin, sg.tile_end, false, dt_fixed, dtbits, 0,
+                                                     sg.tile);
+      else
+        rc = dt ? force_segment<R, true>(g, sg, sg.waves, in_loop, dt_fixed, dtbits, update_hist)
                 : force_segment<R, false>(g, sg, sg.waves, in_loop, dt_fixed, dtbits, update_hist);
+      ++s;
+    }
     if (rc) return rc;
   }
   return 0;
@@ -3030,7 +3436,8 @@ int build_element_tiles(ft_engine *g) {
       int j = i + 1;
       while (j < sg.end && j - i < cap && inst_of_elem[g->perm[j]] == inst) ++j;
       const bool shadow_ok = seg_shadows && i > sg.begin && inst_of_elem[g->perm[i - 1]] == inst;
-      et.push_back(make_int4(i, j, inst, (seg_shadows ? kTileShadows : 0) | (shadow_ok ? kTileShadow : 0)));
+      et.push_back(make_int4(i, j, inst, (seg_shadows ? kTileShadows : 0) | (shadow_ok ? kTileShadow : 0) |
+                                             (sg.mat << kTileMat)));
       i = j;
     }
     sg.tile_end = (int)et.size();
