@@ -1,7 +1,7 @@
 // ft_surrogate.hip -- the constitutive surrogate network on the matrix cores
 // (no counterpart in the reference).
 //
-//   k_mlp_infer  all five layers of a 64-sample slab per wavefront in one
+//   k_mlp_infer  all five layers of a 32-sample slab per wavefront in one
 //                launch: BF16 operands on v_mfma_f32_32x32x16_bf16, FP32
 //                accumulation, bias and SiLU on the accumulators, and the
 //                layer-to-layer hand-over kept in registers (the weights of
@@ -137,24 +137,32 @@ __device__ inline void act_chain(const f32x16 (&acc)[4], bf16x8 (&B)[8]) {
       for (int r = 0; r < 4; ++r) B[2 * t + (j >> 1)][(j & 1) * 4 + r] = (__bf16)silu_fast(acc[t][4 * j + r]);
 }
 
-// y[n][8] = network(x[n][16]).  Persistent blocks of 4 wavefronts: the
-// block stages all weights (BF16, 108 KB) and biases in LDS once, then each
-// wavefront walks 64-sample slabs (two column tiles), the A operands coming
-// from LDS.
-// NT column tiles of 32 samples per wavefront, THREADS per block.  Two
-// tiles at one wavefront per SIMD measured fastest: one tile at two or four
-// wavefronts per SIMD reads every weight fragment from LDS once per tile and
-// ran 25 % slower.
-constexpr int kInferTiles = 2;
-constexpr int kInferThreads = 256;
+// y[n][8] = network(x[n][16]).  Persistent blocks of 8 wavefronts: the
+// block stages all weights (BF16, 117 KB) and biases in LDS once, then each
+// wavefront walks 32-sample slabs, the A operands coming from LDS.
+// NT column tiles of 32 samples per wavefront, THREADS per block: one tile at
+// two wavefronts per SIMD, so that the SiLU evaluations of one overlap the
+// matrix products of the other.  Weight rows in LDS are padded by 16 bytes:
+// the 8 rows of one phase of a 16-byte read then fall on different banks
+// (unpadded, 256-byte rows put them all on the same four, and each fragment
+// read took eight turns).  1.40M samples: 381 us unpadded with two tiles at one
+// wavefront per SIMD, 321 us padded, 244 us with one tile at two (0.60 PFLOP/s;
+// two tiles at two, with spills: 15 us slower).
+constexpr int kInferTiles = 1;
+constexpr int kInferThreads = 512;
+constexpr int kPadIn = kMlpIn + 8, kPadW = kMlpHid + 8;
+constexpr int kWiLds = kMlpHid * kPadIn + (3 * kMlpHid + 32) * kPadW;
 
 template <int NT, int THREADS>
 __global__ __launch_bounds__(THREADS) void k_mlp_infer(const __bf16 *x, long n, const __bf16 *wi, const float *P,
                                                        float *y) {
-  __shared__ __attribute__((aligned(16))) __bf16 sw[kWi];
+  __shared__ __attribute__((aligned(16))) __bf16 sw[kWiLds];
   __shared__ float sb[kMlpLayers * kMlpHid];
-  for (int i = threadIdx.x; i < kWi / 8; i += blockDim.x)
-    reinterpret_cast<bf16x8 *>(sw)[i] = reinterpret_cast<const bf16x8 *>(wi)[i];
+  for (int i = threadIdx.x; i < wi_off(1) / 8; i += blockDim.x)
+    *reinterpret_cast<bf16x8 *>(sw + i / 2 * kPadIn + i % 2 * 8) = reinterpret_cast<const bf16x8 *>(wi)[i];
+  for (int i = threadIdx.x; i < (kWi - wi_off(1)) / 8; i += blockDim.x)
+    *reinterpret_cast<bf16x8 *>(sw + kMlpHid * kPadIn + i / 16 * kPadW + i % 16 * 8) =
+        reinterpret_cast<const bf16x8 *>(wi + wi_off(1))[i];
   for (int i = threadIdx.x; i < kMlpLayers * kMlpHid; i += blockDim.x) {
     const int l = i / kMlpHid, r = i % kMlpHid;
     sb[i] = r < layer_out(l) ? P[b_off(l) + r] : 0.0f;
@@ -181,7 +189,7 @@ __global__ __launch_bounds__(THREADS) void k_mlp_infer(const __bf16 *x, long n, 
       for (int t = 0; t < 4; ++t) acc[c][t] = acc[0][t];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(sw + (32 * t + c32) * kMlpIn + 8 * h);
+      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(sw + (32 * t + c32) * kPadIn + 8 * h);
 #pragma unroll
       for (int c = 0; c < NT; ++c) acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[c][0], acc[c][t], 0, 0, 0);
     }
@@ -189,7 +197,7 @@ __global__ __launch_bounds__(THREADS) void k_mlp_infer(const __bf16 *x, long n, 
     for (int c = 0; c < NT; ++c) act_chain(acc[c], B[c]);
 #pragma unroll 1
     for (int l = 1; l < kMlpLayers - 1; ++l) {
-      const __bf16 *w = sw + wi_off(l);
+      const __bf16 *w = sw + kMlpHid * kPadIn + (l - 1) * kMlpHid * kPadW;
       bias_init(acc[0], sb + l * kMlpHid, h);
 #pragma unroll
       for (int c = 1; c < NT; ++c)
@@ -201,7 +209,7 @@ __global__ __launch_bounds__(THREADS) void k_mlp_infer(const __bf16 *x, long n, 
       for (int s = 0; s < 8; ++s)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const bf16x8 a = *reinterpret_cast<const bf16x8 *>(w + (32 * t + c32) * kMlpHid + 16 * s + 8 * h);
+          const bf16x8 a = *reinterpret_cast<const bf16x8 *>(w + (32 * t + c32) * kPadW + 16 * s + 8 * h);
 #pragma unroll
           for (int c = 0; c < NT; ++c)
             acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[c][s], acc[c][t], 0, 0, 0);
@@ -209,13 +217,13 @@ __global__ __launch_bounds__(THREADS) void k_mlp_infer(const __bf16 *x, long n, 
 #pragma unroll
       for (int c = 0; c < NT; ++c) act_chain(acc[c], B[c]);
     }
-    const __bf16 *w = sw + wi_off(kMlpLayers - 1);
+    const __bf16 *w = sw + kMlpHid * kPadIn + (kMlpLayers - 2) * kMlpHid * kPadW;
     f32x16 o[NT];
 #pragma unroll
     for (int c = 0; c < NT; ++c) o[c] = zero16;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(w + c32 * kMlpHid + 16 * s + 8 * h);
+      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(w + c32 * kPadW + 16 * s + 8 * h);
 #pragma unroll
       for (int c = 0; c < NT; ++c) o[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[c][s], o[c], 0, 0, 0);
     }
