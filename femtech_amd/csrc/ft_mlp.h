@@ -35,10 +35,9 @@ int mlp_infer(MlpNet *net, const __bf16 *x, long n, float *y, hipStream_t st);
 // gradient in the net's gradient vector and the loss in *loss (host).
 int mlp_gradients(MlpNet *net, const __bf16 *x, const float *t, int n, hipStream_t st, double *loss);
 int mlp_copy_gradients(MlpNet *net, float *host);
-// One Adam step with the current gradient (lr, beta1 0.9, beta2 0.999).
-int mlp_adam(MlpNet *net, float lr, hipStream_t st);
 // Batches drawn on the device from a data set (x [n_data][16] BF16,
-// t [n_data][8]); `steps` Adam steps with a cosine-decayed rate.
+// t [n_data][8]); `steps` Adam steps (beta1 0.9, beta2 0.999) with a
+// cosine-decayed rate.
 int mlp_train(MlpNet *net, const __bf16 *x, const float *t, long n_data, int steps, int batch, float lr,
               unsigned long long seed, hipStream_t st, double *final_loss);
 

@@ -8,10 +8,10 @@
 //                layers 1-4 are stored with their input columns permuted to
 //                the accumulator layout, so one layer's output tile is the
 //                next layer's B operand as it stands).
-//   k_gemm       general BF16 MFMA product C = A B with strided operands and
-//                split-K partials (training: forward, input and weight
-//                gradients).
-//   elementwise  bias + SiLU, loss, SiLU backward, column sums, Adam.
+//   k_mlp_train  forward, loss and backward of 128 samples per block in one
+//                launch, leaving every layer's activations and dZ.
+//   k_mlp_grad   weight gradients per 256 samples, bias gradients.
+//   k_mlp_update gradients summed, Adam, BF16 weight copies.
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -79,15 +79,31 @@ __host__ __device__ inline int chain_feature(int kpos) {
   return 32 * (s >> 1) + 16 * (s & 1) + 8 * (pp >> 2) + 4 * h + (pp & 3);
 }
 
-__device__ inline float silu(float z) { return z / (1.0f + __expf(-z)); }
-__device__ inline float silu_grad(float z) {
-  const float s = 1.0f / (1.0f + __expf(-z));
-  return s * (1.0f + z * (1.0f - s));
+// Training copies (BF16): weights as they stand (Pb, the parameter layout) and
+// transposed, Wt: layers 1-3 [in][out], layer 4 [in][16] (outputs past 8 zero).
+__host__ __device__ constexpr int wt_off(int l) { return (l - 1) * kMlpHid * kMlpHid; }
+constexpr int kWt = wt_off(4) + kMlpHid * 16;
+
+// Layer of a parameter and its place there.
+__device__ inline int layer_of(int i) {
+  int l = 0;
+  while (l < kMlpLayers - 1 && i >= w_off(l + 1)) ++l;
+  return l;
 }
 
-__global__ void k_refresh(const float *P, __bf16 *Pb, __bf16 *Wi) {
+// The BF16 copies of parameter i (value v).
+__device__ inline void store_copies(int i, float v, __bf16 *Pb, __bf16 *Wt) {
+  Pb[i] = (__bf16)v;
+  const int l = layer_of(i);
+  if (l == 0 || i >= b_off(l)) return;
+  const int row = (i - w_off(l)) / kMlpHid, col = (i - w_off(l)) % kMlpHid;
+  Wt[wt_off(l) + col * (l == kMlpLayers - 1 ? 16 : kMlpHid) + row] = (__bf16)v;
+}
+
+__global__ void k_refresh(const float *P, __bf16 *Pb, __bf16 *Wi, __bf16 *Wt) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < kParams) Pb[i] = (__bf16)P[i];
+  if (i < kParams) store_copies(i, P[i], Pb, Wt);
+  if (i < kMlpHid * 8) Wt[wt_off(4) + (i / 8) * 16 + 8 + i % 8] = (__bf16)0.0f;
   if (i < kWi) {
     int l, row, col;
     if (i < wi_off(1)) {
@@ -243,128 +259,6 @@ __global__ __launch_bounds__(THREADS) void k_mlp_infer(const __bf16 *x, long n, 
   }
 }
 
-// C (+ blockIdx.y partial) [M][ldc] = A[M][K] B[K][N] over depths
-// [blockIdx.y kchunk, +kchunk); A(m, k) = A[m sam + k sak], B(k, n) =
-// B[k sbk + n sbn].  One 32x32 tile per wavefront.
-struct GemmArgs {
-  int M, N, K;
-  const __bf16 *A;
-  long sam, sak;
-  const __bf16 *B;
-  long sbk, sbn;
-  float *C;
-  int ldc;
-  int kchunk;
-};
-
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
-  const int lane = threadIdx.x & 63, h = lane >> 5, c32 = lane & 31;
-  const int tilesN = (g.N + 31) / 32, tilesM = (g.M + 31) / 32;
-  const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (tile >= tilesM * tilesN) return;  // uniform over the wavefront
-  const int m0 = (tile / tilesN) * 32, n0 = (tile % tilesN) * 32;
-  const int kb = blockIdx.y * g.kchunk, ke = min(g.K, kb + g.kchunk);
-  const int m = m0 + c32, n = n0 + c32;
-  f32x16 acc = {};
-  for (int k0 = kb; k0 < ke; k0 += 16) {
-    bf16x8 a, b;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int k = k0 + 8 * h + i;
-      a[i] = (m < g.M && k < ke) ? g.A[m * g.sam + k * g.sak] : (__bf16)0.0f;
-      b[i] = (n < g.N && k < ke) ? g.B[k * g.sbk + n * g.sbn] : (__bf16)0.0f;
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-  }
-  float *C = g.C + (size_t)blockIdx.y * g.M * g.ldc;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + 8 * j + 4 * h + r;
-      if (row < g.M && n < g.N) C[(size_t)row * g.ldc + n] = acc[4 * j + r];
-    }
-}
-
-// out[i] = sum_z parts[z count + i], z in order (deterministic split-K).
-__global__ void k_sum_parts(const float *parts, int nz, long count, float *out) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  float s = 0.0f;
-  for (int z = 0; z < nz; ++z) s += parts[(size_t)z * count + i];
-  out[i] = s;
-}
-
-// Z[n][w] += b; A = BF16(SiLU(Z)) when act, else A = nothing.
-__global__ void k_bias_act(float *Z, const float *b, long n, int w, int act, __bf16 *A) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * w) return;
-  const float z = Z[i] + b[i % w];
-  Z[i] = z;
-  if (act) A[i] = (__bf16)silu(z);
-}
-
-// Mean squared error over the 6 used outputs: per-block partial sums of
-// (y - t)^2, dY = 2 (y - t) / (6 n) (FP32 and BF16).
-__global__ void k_loss(const float *Y, const float *T, long n, float *dY, __bf16 *dYb, double *part) {
-  __shared__ double sh[256];
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  double e2 = 0.0;
-  if (i < n * kMlpOut) {
-    const int k = (int)(i % kMlpOut);
-    float d = 0.0f;
-    if (k < kMlpUsedOut) {
-      const float r = Y[i] - T[i];
-      e2 = (double)r * r;
-      d = 2.0f * r / (float)(kMlpUsedOut * n);
-    }
-    dY[i] = d;
-    dYb[i] = (__bf16)d;
-  }
-  sh[threadIdx.x] = e2;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-// dZ = dA * SiLU'(Z) (FP32 and BF16).
-__global__ void k_act_bwd(const float *dA, const float *Z, long count, float *dZ, __bf16 *dZb) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const float d = dA[i] * silu_grad(Z[i]);
-  dZ[i] = d;
-  dZb[i] = (__bf16)d;
-}
-
-// db[c] = sum_s dZ[s][c], one block per column, fixed order.
-__global__ void k_colsum(const float *dZ, long n, int w, float *db) {
-  __shared__ float sh[256];
-  const int c = blockIdx.x;
-  float s = 0.0f;
-  for (long i = threadIdx.x; i < n; i += blockDim.x) s += dZ[i * w + c];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) db[c] = sh[0];
-}
-
-__global__ void k_adam(float *P, const float *G, float *m, float *v, float lr, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= kParams) return;
-  const float g = G[i];
-  const float mi = 0.9f * m[i] + 0.1f * g;
-  const float vi = 0.999f * v[i] + 0.001f * g * g;
-  m[i] = mi;
-  v[i] = vi;
-  P[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + 1e-8f);
-}
-
 __device__ inline uint64_t mix64(uint64_t z) {
   z += 0x9E3779B97F4A7C15ull;
   z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -372,16 +266,363 @@ __device__ inline uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-// Batch of `batch` samples drawn uniformly (with replacement) from the data.
-__global__ void k_gather_batch(const __bf16 *x, const float *t, long n_data, int batch, uint64_t key, __bf16 *xb,
-                               float *tb) {
+// ---------------------------------------------------------------------------
+// Training
+// ---------------------------------------------------------------------------
+// k_mlp_train: one block takes 128 samples through forward, loss and backward:
+// 4 wavefronts of 32 samples each, one per SIMD, every product with W^T-shaped
+// A operands from LDS (rows padded by 16 bytes, as in k_mlp_infer) against the
+// wavefront's own samples as B operands, so activations and their gradients
+// pass from layer to layer in registers (the whole register file; SiLU' of the
+// first layer in LDS): an output tile's accumulators (lane half h: rows 8 j +
+// 4 h + r) become B operands (depth 8 h + i) by one v_permlane32_swap per
+// packed pair.  The barriers only guard the weights' two buffers.  For the
+// weight gradients, whose depth is the samples, activations and dZ go to
+// memory sample-contiguous; k_mlp_grad spreads their 56 tiles per 256 samples
+// over the chip.  Every sum keeps its order: products in steps of 16, weight
+// gradients in blocks of 256 samples added in order, bias gradients by 256
+// strided sums and a tree, so a step does not depend on how samples are
+// spread over blocks.
+// A step is a chain of small products: bound by latency and by the SiLU
+// evaluations, not by the matrix cores.  As 37 launches of single products and
+// elementwise passes it took 540 us at a batch of 4,096; as three, 85 us
+// (64 + 15 + 5).
+constexpr int kTrainTile = 128;     // samples per block
+constexpr int kTrainThreads = 256;  // 4 wavefronts x 32 samples
+constexpr int kGradChunk = 256;     // samples per weight-gradient block
+constexpr int kAtRows = kMlpIn + 4 * kMlpHid, kDzRows = 4 * kMlpHid + kMlpOut;
+
+struct TrainArgs {
+  const __bf16 *x;      // [n_data][16]
+  const float *t;       // [n_data][8]
+  long n_data;          // > 0: samples drawn by `key`; 0: sample i of the batch is row i
+  uint64_t key;
+  int n;                // batch size
+  size_t ld;            // samples rounded up to kGradChunk
+  const __bf16 *Pb, *Wt;
+  const float *P;
+  __bf16 *at;           // activations [input 16, layers 1-4 128 each][ld]; zero past n
+  __bf16 *dzb;          // dZ of layers 0-4 (128, ..., 8 rows) [ld], BF16 and FP32; zero past n
+  float *dz;
+  double *lpart;        // squared errors by block
+};
+
+// Accumulators of a 32-row tile (rows 8 j + 4 h + r) as the two B operands of
+// its 16-deep steps (depth 8 h + i), BF16.
+__device__ __forceinline__ void tile_to_operands(const float (&v)[16], bf16x8 (&B)[2]) {
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    unsigned a[2], b[2];  // rows 16 q + 4 h + {0..3}, 16 q + 8 + 4 h + {0..3}
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      bf16x2 lo = {(__bf16)v[8 * q + 2 * k], (__bf16)v[8 * q + 2 * k + 1]};
+      bf16x2 hi = {(__bf16)v[8 * q + 4 + 2 * k], (__bf16)v[8 * q + 4 + 2 * k + 1]};
+      a[k] = __builtin_bit_cast(unsigned, lo);
+      b[k] = __builtin_bit_cast(unsigned, hi);
+    }
+    // upper half of a <-> lower half of b
+    unsigned o[4];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const auto r = __builtin_amdgcn_permlane32_swap(a[k], b[k], false, false);
+      o[k] = r[0];
+      o[2 + k] = r[1];
+    }
+    struct Four { unsigned u[4]; };
+    B[q] = __builtin_bit_cast(bf16x8, Four{{o[0], o[1], o[2], o[3]}});
+  }
+}
+
+// SiLU and its derivative as z / (1 + e^-z) and s (1 + z (1 - s)), s = 1 / (1 +
+// e^-z): the reciprocal refined to full precision serves both divisions.
+__device__ __forceinline__ void silu_both(float z, float &v, float &d) {
+  const float ez = 1.0f + __expf(-z);
+  float s = __builtin_amdgcn_rcpf(ez);
+  const float r = fmaf(fmaf(-ez, s, 1.0f), s, s);
+  s = ez < 1e30f ? r : 0.0f;  // (beyond, both vanish in FP32)
+  const float q = z * s;
+  v = ez < 1e30f ? fmaf(fmaf(-q, ez, z), s, q) : z * 0.0f;
+  d = s * (1.0f + z * (1.0f - s));
+}
+
+// The products of a layer: acc[t] = sum_k W(32 t + c32, 16 k + ..) B[k], weight
+// rows at `wl` (LDS, row stride kPadW).
+template <int STEPS>
+__device__ __forceinline__ void layer_product(const __bf16 *wl, int c32, int h, const bf16x8 (&B)[8], f32x16 (&acc)[4]) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = f32x16{};
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(wl + (32 * t + c32) * kPadW + 16 * k + 8 * h);
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[k], acc[t], 0, 0, 0);
+    }
+}
+
+struct TrainLds {
+  __attribute__((aligned(16))) __bf16 w[2][kMlpHid * kPadW];  // weights of this layer and the next
+  float zg0[4][64][64];                                       // SiLU'(Z_0) by wavefront and lane
+  float b[kMlpLayers * kMlpHid];                              // biases
+  double loss[4];
+};
+
+__global__ __launch_bounds__(kTrainThreads) void k_mlp_train(TrainArgs g) {
+  __shared__ TrainLds lds;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, c32 = lane & 31;
+  const size_t i = (size_t)blockIdx.x * kTrainTile + 32 * w + c32;  // sample in the batch (below ld)
+  const bool valid = i < (size_t)g.n;
+  const bf16x8 zero8 = {};
+  // weights of a product: rows x 128 (or 16) deep, 16 bytes per thread and turn, through registers
+  constexpr int kTurns = kMlpHid * kMlpHid / 8 / kTrainThreads;
+  bf16x8 pre[kTurns];
+  auto fetch = [&](const __bf16 *src, int chunks) {
+#pragma unroll
+    for (int k = 0; k < kTurns; ++k) {
+      const int c = k * kTrainThreads + (int)threadIdx.x;
+      if (c < chunks) pre[k] = reinterpret_cast<const bf16x8 *>(src)[c];
+    }
+  };
+  auto stage = [&](int buf, int chunks, int per_row) {
+#pragma unroll
+    for (int k = 0; k < kTurns; ++k) {
+      const int c = k * kTrainThreads + (int)threadIdx.x;
+      if (c < chunks) *reinterpret_cast<bf16x8 *>(&lds.w[buf][(c / per_row) * kPadW + (c % per_row) * 8]) = pre[k];
+    }
+  };
+  constexpr int kFull = kMlpHid * kMlpHid / 8, kIn = kMlpHid * kMlpIn / 8, kOut = kMlpOut * kMlpHid / 8;
+  constexpr int kOutT = kMlpHid * 16 / 8;
+  fetch(g.Pb + w_off(0), kIn);
+  for (int k = threadIdx.x; k < kMlpLayers * kMlpHid; k += kTrainThreads) {
+    const int l = k / kMlpHid, r = k % kMlpHid;
+    lds.b[k] = r < layer_out(l) ? g.P[b_off(l) + r] : 0.0f;
+  }
+  size_t row = i;
+  if (g.n_data > 0) row = (size_t)(mix64(g.key ^ (uint64_t)i * 0xD1B54A32D192ED03ull) % (uint64_t)g.n_data);
+  bf16x8 B[8];
+  B[0] = valid ? *reinterpret_cast<const bf16x8 *>(g.x + row * kMlpIn + 8 * h) : zero8;
+  const float4 tv = valid ? *reinterpret_cast<const float4 *>(g.t + row * kMlpOut + 4 * h) : float4{0, 0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 8; ++k) g.at[(8 * h + k) * g.ld + i] = B[0][k];
+  stage(0, kIn, kMlpIn / 8);
+  fetch(g.Pb + w_off(1), kFull);
+  __syncthreads();
+  // ---- forward: Z_l = W_l A_{l-1} + b_l, A_l = SiLU(Z_l); layer l's weights are in buffer l % 2
+  float zg[3][64];  // SiLU'(Z_l), l = 1-3
+  f32x16 acc[4];
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    if (l == 0)
+      layer_product<1>(lds.w[0], c32, h, B, acc);
+    else
+      layer_product<8>(lds.w[l & 1], c32, h, B, acc);
+    __bf16 *al = g.at + (size_t)(kMlpIn + l * kMlpHid) * g.ld + i;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float v[16];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int f = 32 * t + 8 * j + 4 * h;
+        const float4 b4 = *reinterpret_cast<const float4 *>(&lds.b[l * kMlpHid + f]);
+        const float bb[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int e = 4 * j + r;
+          float d;
+          silu_both(acc[t][e] + bb[r], v[e], d);
+          if (l == 0)
+            lds.zg0[w][16 * t + e][lane] = d;
+          else
+            zg[l - 1][16 * t + e] = d;
+          al[(size_t)(f + r) * g.ld] = valid ? (__bf16)v[e] : (__bf16)0.0f;
+        }
+      }
+      bf16x8 two[2];
+      tile_to_operands(v, two);
+      B[2 * t] = two[0];
+      B[2 * t + 1] = two[1];
+    }
+    // the next layer's weights into the other buffer (its last readers passed the barrier before)
+    if (l < 3)
+      stage((l + 1) & 1, kFull, kMlpHid / 8);
+    else
+      stage(0, kOut, kMlpHid / 8);
+    if (l < 2)
+      fetch(g.Pb + w_off(l + 2), kFull);
+    else if (l == 2)
+      fetch(g.Pb + w_off(4), kOut);
+    else
+      fetch(g.Wt + wt_off(4), kOutT);
+    __syncthreads();
+  }
+  // ---- output layer, loss: mean squared error over the 6 used outputs
+  f32x16 o = {};
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const bf16x8 a =
+        c32 < kMlpOut ? *reinterpret_cast<const bf16x8 *>(&lds.w[0][c32 * kPadW + 16 * k + 8 * h]) : zero8;
+    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[k], o, 0, 0, 0);
+  }
+  stage(1, kOutT, 2);  // W4^T (layer 3's weights were last read before the barrier)
+  fetch(g.Wt + wt_off(3), kFull);
+  float dy[4];
+  double e2 = 0.0;
+  {
+    const float tt[4] = {tv.x, tv.y, tv.z, tv.w};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = 4 * h + r;
+      const float d = (o[r] + lds.b[4 * kMlpHid + k]) - tt[r];
+      const bool use = valid && k < kMlpUsedOut;
+      dy[r] = use ? 2.0f * d / (float)(kMlpUsedOut * (long)g.n) : 0.0f;
+      if (use) e2 += (double)d * d;
+    }
+  }
+  for (int m = 32; m > 0; m >>= 1) e2 += __shfl_xor(e2, m);
+  if (lane == 0) lds.loss[w] = e2;
+  // dZ of the output layer: to memory, and as the B operand (depth 8: the lower half holds all 8)
+  B[0] = zero8;
+  {
+    float other[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) other[r] = __shfl_xor(dy[r], 32);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      B[0][r] = h ? (__bf16)0.0f : (__bf16)dy[r];
+      B[0][4 + r] = h ? (__bf16)0.0f : (__bf16)other[r];
+      const size_t at = (size_t)(4 * kMlpHid + 4 * h + r) * g.ld + i;
+      g.dz[at] = dy[r];
+      g.dzb[at] = (__bf16)dy[r];
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) g.lpart[blockIdx.x] = lds.loss[0] + lds.loss[1] + lds.loss[2] + lds.loss[3];
+  // ---- backward: dA_{l-1} = W_l^T dZ_l (W_l^T in buffer (l + 1) % 2); dZ_{l-1} = dA SiLU'(Z_{l-1})
+#pragma unroll
+  for (int l = 4; l >= 1; --l) {
+    if (l == 4)
+      layer_product<1>(lds.w[1], c32, h, B, acc);
+    else
+      layer_product<8>(lds.w[(l + 1) & 1], c32, h, B, acc);
+    if (l > 1) {
+      stage(l & 1, kFull, kMlpHid / 8);  // W_{l-1}^T
+      if (l > 2) fetch(g.Wt + wt_off(l - 2), kFull);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float v[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const size_t at = (size_t)((l - 1) * kMlpHid + 32 * t + 8 * (e >> 2) + 4 * h + (e & 3)) * g.ld + i;
+        const float d = l == 1 ? lds.zg0[w][16 * t + e][lane] : zg[l > 1 ? l - 2 : 0][16 * t + e];
+        v[e] = valid ? acc[t][e] * d : 0.0f;
+        g.dz[at] = v[e];
+        g.dzb[at] = (__bf16)v[e];
+      }
+      if (l > 1) {
+        bf16x8 two[2];
+        tile_to_operands(v, two);
+        B[2 * t] = two[0];
+        B[2 * t + 1] = two[1];
+      }
+    }
+    if (l > 1) __syncthreads();
+  }
+}
+
+// Weight and bias gradients from k_mlp_train's arrays.  Blocks (x, z): x < 14:
+// weight gradients of samples [256 z, + 256), dW_l[o][i] = sum_s dZ_l[o][s]
+// A_{l-1}[i][s], a 32x32 tile per wavefront (layer 0: x 0, one output tile per
+// wavefront; layers 1-3: x 1-12, an output tile each, an input tile per
+// wavefront; layer 4: x 13), into parts[z].  x >= 14 (z = 0): the bias
+// gradients, one row of dZ each, summed in a fixed order into db.
+constexpr int kGradTiles = 14;
+__global__ __launch_bounds__(256) void k_mlp_grad(const __bf16 *at, const __bf16 *dzb, const float *dz, size_t ld,
+                                                  float *parts, float *db) {
+  const int x = blockIdx.x, w = threadIdx.x >> 6;
+  if (x >= kGradTiles) {
+    if (blockIdx.y) return;
+    __shared__ float sh[256];
+    const float *src = dz + (size_t)(x - kGradTiles) * ld;
+    float q = 0.0f;
+    for (size_t k = threadIdx.x; k < ld; k += 256) q += src[k];
+    sh[threadIdx.x] = q;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+      if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) db[x - kGradTiles] = sh[0];
+    return;
+  }
+  const int l = x == 0 ? 0 : (x == 13 ? 4 : 1 + (x - 1) / 4);
+  const int ot = x == 0 ? w : (x == 13 ? 0 : (x - 1) % 4), it = x == 0 ? 0 : w;
+  const int in = layer_in(l), out = layer_out(l);
+  const int lane = threadIdx.x & 63, h = lane >> 5, c32 = lane & 31;
+  const int r = 32 * ot + c32, c = 32 * it + c32;
+  const size_t s0 = (size_t)blockIdx.y * kGradChunk + 8 * h;
+  const __bf16 *ap = dzb + (size_t)(l * kMlpHid + r) * ld + s0;
+  const __bf16 *bp = at + (size_t)((l == 0 ? 0 : kMlpIn + (l - 1) * kMlpHid) + c) * ld + s0;
+  const bf16x8 zero8 = {};
+  bf16x8 a[kGradChunk / 16], b[kGradChunk / 16];
+#pragma unroll
+  for (int k = 0; k < kGradChunk / 16; ++k) {
+    a[k] = r < out ? *reinterpret_cast<const bf16x8 *>(ap + 16 * k) : zero8;
+    b[k] = c < in ? *reinterpret_cast<const bf16x8 *>(bp + 16 * k) : zero8;
+  }
+  f32x16 acc = {};
+#pragma unroll
+  for (int k = 0; k < kGradChunk / 16; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], b[k], acc, 0, 0, 0);
+  if (c >= in) return;
+  float *dst = parts + (size_t)blockIdx.y * kParams + w_off(l) + c;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int o = 32 * ot + 8 * (e >> 2) + 4 * h + (e & 3);
+    if (o < out) dst[o * in] = acc[e];
+  }
+}
+
+// Gradients: the weights' parts added in order, the biases' as they are; with
+// `adam`, the parameter update and its BF16 copies.
+__global__ void k_mlp_update(const float *parts, int nz, const float *db, float *G, int adam, float *P, float *m,
+                             float *v, float lr, float c1, float c2, __bf16 *Pb, __bf16 *Wt) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= batch) return;
-  const long s = (long)(mix64(key ^ (uint64_t)i * 0xD1B54A32D192ED03ull) % (uint64_t)n_data);
-  *reinterpret_cast<bf16x8 *>(xb + (size_t)i * kMlpIn) = *reinterpret_cast<const bf16x8 *>(x + s * kMlpIn);
-  *reinterpret_cast<bf16x8 *>(xb + (size_t)i * kMlpIn + 8) = *reinterpret_cast<const bf16x8 *>(x + s * kMlpIn + 8);
-  *reinterpret_cast<float4 *>(tb + (size_t)i * kMlpOut) = *reinterpret_cast<const float4 *>(t + s * kMlpOut);
-  *reinterpret_cast<float4 *>(tb + (size_t)i * kMlpOut + 4) = *reinterpret_cast<const float4 *>(t + s * kMlpOut + 4);
+  if (i >= kParams) return;
+  const int l = layer_of(i);
+  float g = 0.0f;
+  if (i >= b_off(l)) {
+    g = db[l * kMlpHid + i - b_off(l)];
+  } else {
+    int z = 0;
+    for (; z + 8 <= nz; z += 8) {  // 8 loads in flight
+      float q[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) q[k] = parts[(size_t)(z + k) * kParams + i];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) g += q[k];
+    }
+    for (; z < nz; ++z) g += parts[(size_t)z * kParams + i];
+  }
+  G[i] = g;
+  if (!adam) return;
+  const float mi = 0.9f * m[i] + 0.1f * g;
+  const float vi = 0.999f * v[i] + 0.001f * g * g;
+  m[i] = mi;
+  v[i] = vi;
+  const float p = P[i] - lr * (mi * c1) / (sqrtf(vi * c2) + 1e-8f);
+  P[i] = p;
+  store_copies(i, p, Pb, Wt);
+}
+
+__global__ void k_to_bf16(const float *x, size_t n, __bf16 *y) {
+  const size_t i = 4 * ((size_t)blockIdx.x * blockDim.x + threadIdx.x);
+  if (i >= n) return;  // n is a multiple of 16
+  const float4 v = *reinterpret_cast<const float4 *>(x + i);
+  y[i] = (__bf16)v.x;
+  y[i + 1] = (__bf16)v.y;
+  y[i + 2] = (__bf16)v.z;
+  y[i + 3] = (__bf16)v.w;
 }
 
 int blocks(long n, int b = 256) { return (int)((n + b - 1) / b); }
@@ -390,80 +631,86 @@ int blocks(long n, int b = 256) { return (int)((n + b - 1) / b); }
 
 struct MlpNet {
   float *P = nullptr, *G = nullptr, *m = nullptr, *v = nullptr;
-  __bf16 *Pb = nullptr, *Wi = nullptr;
+  __bf16 *Pb = nullptr, *Wi = nullptr, *Wt = nullptr;
+  bool wi_stale = false;  // Wi (inference) is behind P
   int adam_t = 0;
   int n_cu = 0;  // compute units (persistent inference grid)
-  // training workspace for batches up to `cap` samples
-  int cap = 0;
-  float *Z[kMlpLayers] = {};
-  __bf16 *A[kMlpLayers - 1] = {};
-  float *dZ = nullptr, *dA = nullptr, *parts = nullptr;
-  __bf16 *dZb = nullptr, *xb = nullptr;
-  float *tb = nullptr, *dY = nullptr;
-  __bf16 *dYb = nullptr;
+  // training workspace for batches up to `ld` samples
+  size_t ld = 0;
+  __bf16 *at = nullptr, *dzb = nullptr;
+  float *dz = nullptr, *parts = nullptr, *db = nullptr;
   double *lpart = nullptr;
-  size_t parts_len = 0;
 };
 
 namespace {
 
 void free_ws(MlpNet *n) {
-  for (auto &p : n->Z) (void)hipFree(p), p = nullptr;
-  for (auto &p : n->A) (void)hipFree(p), p = nullptr;
-  for (void *p : {(void *)n->dZ, (void *)n->dA, (void *)n->parts, (void *)n->dZb, (void *)n->xb, (void *)n->tb,
-                  (void *)n->dY, (void *)n->dYb, (void *)n->lpart})
+  for (void *p : {(void *)n->at, (void *)n->dzb, (void *)n->dz, (void *)n->parts, (void *)n->db, (void *)n->lpart})
     if (p) (void)hipFree(p);
-  n->dZ = n->dA = n->parts = n->tb = n->dY = nullptr;
-  n->dZb = n->xb = n->dYb = nullptr;
+  n->at = n->dzb = nullptr;
+  n->dz = n->parts = n->db = nullptr;
   n->lpart = nullptr;
-  n->cap = 0;
+  n->ld = 0;
 }
+
+size_t train_ld(int batch) { return ((size_t)batch + kGradChunk - 1) / kGradChunk * kGradChunk; }
 
 int ensure_ws(MlpNet *n, int batch) {
-  if (batch <= n->cap) return 0;
+  const size_t ld = train_ld(batch);
+  if (ld <= n->ld) return 0;
   free_ws(n);
-  const size_t b = (size_t)batch;
-  for (int l = 0; l < kMlpLayers; ++l) MCHK(hipMalloc(&n->Z[l], b * layer_out(l) * sizeof(float)));
-  for (int l = 0; l < kMlpLayers - 1; ++l) MCHK(hipMalloc(&n->A[l], b * layer_out(l) * sizeof(__bf16)));
-  MCHK(hipMalloc(&n->dZ, b * kMlpHid * sizeof(float)));
-  MCHK(hipMalloc(&n->dA, b * kMlpHid * sizeof(float)));
-  MCHK(hipMalloc(&n->dZb, b * kMlpHid * sizeof(__bf16)));
-  MCHK(hipMalloc(&n->xb, b * kMlpIn * sizeof(__bf16)));
-  MCHK(hipMalloc(&n->tb, b * kMlpOut * sizeof(float)));
-  MCHK(hipMalloc(&n->dY, b * kMlpOut * sizeof(float)));
-  MCHK(hipMalloc(&n->dYb, b * kMlpOut * sizeof(__bf16)));
-  MCHK(hipMalloc(&n->lpart, (size_t)blocks(b * kMlpOut) * sizeof(double)));
-  n->parts_len = (size_t)((batch + 255) / 256) * kMlpHid * kMlpHid;
-  MCHK(hipMalloc(&n->parts, n->parts_len * sizeof(float)));
-  n->cap = batch;
-  return 0;
-}
-
-// C[M][ldc] = A B, split over the depth in chunks of `kchunk` when K is long.
-int gemm(MlpNet *net, GemmArgs g, hipStream_t st) {
-  const int tiles = ((g.M + 31) / 32) * ((g.N + 31) / 32);
-  const int nz = (g.K + g.kchunk - 1) / g.kchunk;
-  float *out = g.C;
-  const int ldc = g.ldc;
-  if (nz > 1) {
-    if ((size_t)nz * g.M * g.N > net->parts_len) return mfail(FT_ERR_ARG, "split-K workspace too small");
-    g.C = net->parts;
-    g.ldc = g.N;
-  }
-  hipLaunchKernelGGL(k_gemm, dim3((tiles + 3) / 4, nz), dim3(256), 0, st, g);
-  MCHK(hipGetLastError());
-  if (nz > 1) {
-    if (ldc != g.N) return mfail(FT_ERR_ARG, "split-K output must be dense");
-    const long count = (long)g.M * g.N;
-    hipLaunchKernelGGL(k_sum_parts, dim3(blocks(count)), dim3(256), 0, st, net->parts, nz, count, out);
-    MCHK(hipGetLastError());
-  }
+  MCHK(hipMalloc(&n->at, kAtRows * ld * sizeof(__bf16)));
+  MCHK(hipMalloc(&n->dzb, kDzRows * ld * sizeof(__bf16)));
+  MCHK(hipMalloc(&n->dz, kDzRows * ld * sizeof(float)));
+  MCHK(hipMalloc(&n->parts, ld / kGradChunk * kParams * sizeof(float)));
+  MCHK(hipMalloc(&n->db, kDzRows * sizeof(float)));
+  MCHK(hipMalloc(&n->lpart, ld / kTrainTile * sizeof(double)));
+  n->ld = ld;
   return 0;
 }
 
 int refresh(MlpNet *net, hipStream_t st) {
-  hipLaunchKernelGGL(k_refresh, dim3(blocks(std::max(kParams, kWi))), dim3(256), 0, st, net->P, net->Pb, net->Wi);
+  hipLaunchKernelGGL(k_refresh, dim3(blocks(std::max(kParams, kWi))), dim3(256), 0, st, net->P, net->Pb, net->Wi,
+                     net->Wt);
   MCHK(hipGetLastError());
+  net->wi_stale = false;
+  return 0;
+}
+
+struct AdamStep {
+  float lr, c1, c2;
+};
+
+// One batch: gradients into G and, with `adam`, the parameter update.
+// n_data > 0 draws the batch from (x, t) by `key`, else it is their first n
+// rows.
+int train_batch(MlpNet *net, const __bf16 *x, const float *t, long n_data, uint64_t key, int n, const AdamStep *adam,
+                hipStream_t st) {
+  int rc;
+  if ((rc = ensure_ws(net, n))) return rc;
+  const size_t ld = train_ld(n);
+  const TrainArgs g{x, t, n_data, key, n, ld, net->Pb, net->Wt, net->P, net->at, net->dzb, net->dz, net->lpart};
+  hipLaunchKernelGGL(k_mlp_train, dim3((unsigned)(ld / kTrainTile)), dim3(kTrainThreads), 0, st, g);
+  MCHK(hipGetLastError());
+  const int nz = (int)(ld / kGradChunk);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(kGradTiles + kDzRows, nz), dim3(256), 0, st, net->at, net->dzb, net->dz, ld,
+                     net->parts, net->db);
+  MCHK(hipGetLastError());
+  hipLaunchKernelGGL(k_mlp_update, dim3(blocks(kParams)), dim3(256), 0, st, net->parts, nz, net->db, net->G,
+                     adam ? 1 : 0, net->P, net->m, net->v, adam ? adam->lr : 0.0f, adam ? adam->c1 : 0.0f,
+                     adam ? adam->c2 : 0.0f, net->Pb, net->Wt);
+  MCHK(hipGetLastError());
+  if (adam) net->wi_stale = true;
+  return 0;
+}
+
+int read_loss(MlpNet *net, int n, hipStream_t st, double *loss) {
+  std::vector<double> part(((size_t)n + kTrainTile - 1) / kTrainTile);
+  MCHK(hipMemcpyAsync(part.data(), net->lpart, part.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+  MCHK(hipStreamSynchronize(st));
+  double s = 0.0;
+  for (double p : part) s += p;
+  *loss = s / ((double)n * kMlpUsedOut);
   return 0;
 }
 
@@ -483,7 +730,8 @@ int mlp_create(unsigned long long seed, MlpNet **out) {
       hipMalloc(&n->m, kParams * sizeof(float)) != hipSuccess ||
       hipMalloc(&n->v, kParams * sizeof(float)) != hipSuccess ||
       hipMalloc(&n->Pb, kParams * sizeof(__bf16)) != hipSuccess ||
-      hipMalloc(&n->Wi, kWi * sizeof(__bf16)) != hipSuccess)
+      hipMalloc(&n->Wi, kWi * sizeof(__bf16)) != hipSuccess ||
+      hipMalloc(&n->Wt, kWt * sizeof(__bf16)) != hipSuccess)
     return bail(mfail(FT_ERR_ALLOC, "network allocation failed"));
   // Glorot-uniform weights from a 64-bit mix of (seed, index), zero biases
   std::vector<float> h(kParams, 0.0f);
@@ -510,7 +758,8 @@ void mlp_destroy(MlpNet *n) {
   if (!n) return;
   (void)hipDeviceSynchronize();
   free_ws(n);
-  for (void *p : {(void *)n->P, (void *)n->G, (void *)n->m, (void *)n->v, (void *)n->Pb, (void *)n->Wi})
+  for (void *p : {(void *)n->P, (void *)n->G, (void *)n->m, (void *)n->v, (void *)n->Pb, (void *)n->Wi,
+                  (void *)n->Wt})
     if (p) (void)hipFree(p);
   delete n;
 }
@@ -539,6 +788,8 @@ int mlp_copy_gradients(MlpNet *net, float *host) {
 
 int mlp_infer(MlpNet *net, const __bf16 *x, long n, float *y, hipStream_t st) {
   if (n <= 0) return 0;
+  int rc;
+  if (net->wi_stale && (rc = refresh(net, st))) return rc;
   if (!net->n_cu) {
     int dev = 0;
     MCHK(hipGetDevice(&dev));
@@ -556,87 +807,31 @@ int mlp_infer(MlpNet *net, const __bf16 *x, long n, float *y, hipStream_t st) {
 int mlp_gradients(MlpNet *net, const __bf16 *x, const float *t, int n, hipStream_t st, double *loss) {
   if (n <= 0) return mfail(FT_ERR_ARG, "empty batch");
   int rc;
-  if ((rc = ensure_ws(net, n))) return rc;
-  // forward: Z_l = A_{l-1} W_l^T + b_l, A_l = SiLU(Z_l)
-  const __bf16 *Aprev = x;
-  for (int l = 0; l < kMlpLayers; ++l) {
-    const int in = layer_in(l), out = layer_out(l);
-    GemmArgs g{n, out, in, Aprev, in, 1, net->Pb + w_off(l), 1, in, net->Z[l], out, in};
-    if ((rc = gemm(net, g, st))) return rc;
-    const bool act = l < kMlpLayers - 1;
-    hipLaunchKernelGGL(k_bias_act, dim3(blocks((long)n * out)), dim3(256), 0, st, net->Z[l], net->P + b_off(l),
-                       (long)n, out, act ? 1 : 0, act ? net->A[l] : nullptr);
-    MCHK(hipGetLastError());
-    if (act) Aprev = net->A[l];
-  }
-  const int nb = blocks((long)n * kMlpOut);
-  hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, st, net->Z[kMlpLayers - 1], t, (long)n, net->dY, net->dYb,
-                     net->lpart);
-  MCHK(hipGetLastError());
-  // backward
-  const float *dZ = net->dY;
-  const __bf16 *dZb = net->dYb;
-  for (int l = kMlpLayers - 1; l >= 0; --l) {
-    const int in = layer_in(l), out = layer_out(l);
-    const __bf16 *Ain = l == 0 ? x : net->A[l - 1];
-    // dW_l[o][i] = sum_s dZ[s][o] A_{l-1}[s][i]
-    GemmArgs gw{out, in, n, dZb, 1, out, Ain, in, 1, net->G + w_off(l), in, 256};
-    if ((rc = gemm(net, gw, st))) return rc;
-    hipLaunchKernelGGL(k_colsum, dim3(out), dim3(256), 0, st, dZ, (long)n, out, net->G + b_off(l));
-    MCHK(hipGetLastError());
-    if (l == 0) break;
-    // dA_{l-1}[s][i] = sum_o dZ[s][o] W_l[o][i]; dZ_{l-1} = dA SiLU'(Z_{l-1})
-    GemmArgs gd{n, in, out, dZb, out, 1, net->Pb + w_off(l), in, 1, net->dA, in, out};
-    if ((rc = gemm(net, gd, st))) return rc;
-    hipLaunchKernelGGL(k_act_bwd, dim3(blocks((long)n * in)), dim3(256), 0, st, net->dA, net->Z[l - 1],
-                       (long)n * in, net->dZ, net->dZb);
-    MCHK(hipGetLastError());
-    dZ = net->dZ;
-    dZb = net->dZb;
-  }
-  if (loss) {
-    std::vector<double> part(nb);
-    MCHK(hipMemcpyAsync(part.data(), net->lpart, nb * sizeof(double), hipMemcpyDeviceToHost, st));
-    MCHK(hipStreamSynchronize(st));
-    double s = 0.0;
-    for (double p : part) s += p;
-    *loss = s / ((double)n * kMlpUsedOut);
-  }
-  return 0;
-}
-
-int mlp_adam(MlpNet *net, float lr, hipStream_t st) {
-  net->adam_t += 1;
-  const float c1 = (float)(1.0 / (1.0 - pow(0.9, net->adam_t)));
-  const float c2 = (float)(1.0 / (1.0 - pow(0.999, net->adam_t)));
-  hipLaunchKernelGGL(k_adam, dim3(blocks(kParams)), dim3(256), 0, st, net->P, net->G, net->m, net->v, lr, c1, c2);
-  MCHK(hipGetLastError());
-  return refresh(net, st);
+  if ((rc = train_batch(net, x, t, 0, 0, n, nullptr, st))) return rc;
+  return loss ? read_loss(net, n, st, loss) : 0;
 }
 
 int mlp_train(MlpNet *net, const __bf16 *x, const float *t, long n_data, int steps, int batch, float lr,
               unsigned long long seed, hipStream_t st, double *final_loss) {
   if (n_data <= 0 || batch <= 0 || steps < 0) return mfail(FT_ERR_ARG, "empty training set or batch");
   int rc;
-  if ((rc = ensure_ws(net, batch))) return rc;
   double acc = 0.0;
   int nacc = 0;
   for (int k = 0; k < steps; ++k) {
     const uint64_t key = seed * 0x9E3779B97F4A7C15ull ^ ((uint64_t)k << 20);
-    hipLaunchKernelGGL(k_gather_batch, dim3(blocks(batch)), dim3(256), 0, st, x, t, n_data, batch, key, net->xb,
-                       net->tb);
-    MCHK(hipGetLastError());
+    const float lr_k = lr * (0.02f + 0.98f * 0.5f * (1.0f + cosf(3.14159265f * (float)k / (float)steps)));
+    net->adam_t += 1;
+    const AdamStep a{lr_k, (float)(1.0 / (1.0 - pow(0.9, net->adam_t))), (float)(1.0 / (1.0 - pow(0.999, net->adam_t)))};
+    if ((rc = train_batch(net, x, t, n_data, key, batch, &a, st))) return rc;
     // the loss is read back (a synchronisation) only over the last 1 % of steps
-    const bool read = final_loss && k >= steps - std::max(1, steps / 100);
-    double l = 0.0;
-    if ((rc = mlp_gradients(net, net->xb, net->tb, batch, st, read ? &l : nullptr))) return rc;
-    if (read) {
+    if (final_loss && k >= steps - std::max(1, steps / 100)) {
+      double l = 0.0;
+      if ((rc = read_loss(net, batch, st, &l))) return rc;
       acc += l;
       ++nacc;
     }
-    const float lr_k = lr * (0.02f + 0.98f * 0.5f * (1.0f + cosf(3.14159265f * (float)k / (float)steps)));
-    if ((rc = mlp_adam(net, lr_k, st))) return rc;
   }
+  if (net->wi_stale && (rc = refresh(net, st))) return rc;
   MCHK(hipStreamSynchronize(st));
   if (final_loss) *final_loss = nacc ? acc / nacc : 0.0;
   return 0;
@@ -653,20 +848,25 @@ struct ft_mlp {
 
 namespace {
 
-int to_device_bf16(const float *host, size_t count, __bf16 **dev) {
-  std::vector<__bf16> h(count);
-  for (size_t i = 0; i < count; ++i) h[i] = (__bf16)host[i];
-  if (hipMalloc(dev, count * sizeof(__bf16)) != hipSuccess) return ft::mfail(FT_ERR_ALLOC, "allocation failed");
-  if (hipMemcpy(*dev, h.data(), count * sizeof(__bf16), hipMemcpyHostToDevice) != hipSuccess)
-    return ft::mfail(FT_ERR_HIP, "copy failed");
-  return 0;
-}
-
 int to_device_f32(const float *host, size_t count, float **dev) {
   if (hipMalloc(dev, count * sizeof(float)) != hipSuccess) return ft::mfail(FT_ERR_ALLOC, "allocation failed");
   if (hipMemcpy(*dev, host, count * sizeof(float), hipMemcpyHostToDevice) != hipSuccess)
     return ft::mfail(FT_ERR_HIP, "copy failed");
   return 0;
+}
+
+// Rounded on the device: the host's conversion loop took longer than the copy.
+int to_device_bf16(const float *host, size_t count, __bf16 **dev) {
+  float *f = nullptr;
+  int rc = to_device_f32(host, count, &f);
+  if (!rc && hipMalloc(dev, count * sizeof(__bf16)) != hipSuccess) rc = ft::mfail(FT_ERR_ALLOC, "allocation failed");
+  if (!rc) {
+    hipLaunchKernelGGL(ft::k_to_bf16, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, nullptr, f, count, *dev);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+      rc = ft::mfail(FT_ERR_HIP, "conversion failed");
+  }
+  if (f) (void)hipFree(f);
+  return rc;
 }
 
 int device_ok() {
