@@ -1988,8 +1988,19 @@ constexpr int kInjIncluded = 1, kInjGt15 = 2, kInjGt30 = 4, kInjPsr120 = 8, kInj
 constexpr int kInjMps95 = 32, kInjMpsxsr95 = 64;
 // Running scalars: (value, original element id, time) for max principal,
 // min principal, max shear and max PS x SR; (value, time) for MPS-95 and
-// MPSxSR-95; then two "list needs refresh" flags.
+// MPSxSR-95; then two unused and the MPS-95 / MPSxSR-95 maxima before this
+// update (kInjOld).
 constexpr int kInjScal = 20;
+constexpr int kInjOld = 18;
+// Digits of the percentile search (k_select_hist): bits of the first digit,
+// of the others, and their count.
+constexpr int kSelFirst = 9, kSelBits = 11, kSelPasses = 6;
+static_assert(kSelFirst + (kSelPasses - 1) * kSelBits == 64, "digits of a 64-bit key");
+__host__ __device__ constexpr int sel_bins(int pass) { return 1 << (pass == 0 ? kSelFirst : kSelBits); }
+__host__ __device__ constexpr int sel_base(int pass) {  // first counter of a pass (2 arrays of bins each)
+  return pass == 0 ? 0 : 2 * (sel_bins(0) + (pass - 1) * sel_bins(1));
+}
+__host__ __device__ constexpr int sel_shift(int pass) { return 64 - kSelFirst - pass * kSelBits; }
 struct InjuryArgs {
   int nn, ne;
   const int *conn;
@@ -1999,6 +2010,7 @@ struct InjuryArgs {
   double *ps_old, *psxsr;
   double *part;      // 8 doubles per block
   double *scal;      // kInjScal
+  unsigned *hist;    // sel_base(kSelPasses) counters
   const StepSlot *slot;  // time / dt source (nullable: use time, dt)
   double time, dt;
 };
@@ -2032,12 +2044,26 @@ __device__ inline ArgBest block_argbest(ArgBest x, bool is_max) {
   return r;
 }
 
+// Order-preserving keys of doubles (NaN above infinity).
+__device__ inline unsigned long long order_key(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
+}
+__device__ inline double key_value(unsigned long long k) {
+  const unsigned long long b = (k >> 63) ? (k & 0x7FFFFFFFFFFFFFFFull) : ~k;
+  return __longlong_as_double((long long)b);
+}
+
 __global__ __launch_bounds__(kBlock) void k_injury_elem(InjuryArgs a) {
   if (a.slot && a.slot->done) return;  // uniform
   const double dt = a.slot ? a.slot->dt : a.dt;
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   const double ninf = -INFINITY;
   ArgBest bmax{ninf, INT32_MAX}, bmin{INFINITY, INT32_MAX}, bsh{ninf, INT32_MAX}, bx{ninf, INT32_MAX};
+  // the first digit of the percentile search on the way (k_select_hist)
+  __shared__ unsigned h[2][sel_bins(0)];
+  for (int i = threadIdx.x; i < 2 * sel_bins(0); i += blockDim.x) (&h[0][0])[i] = 0;
+  __syncthreads();
   if (e < a.ne && (a.flags[e] & kInjIncluded)) {
     int nd[8];
     for (int k = 0; k < 8; ++k) nd[k] = a.conn[8 * (size_t)e + k];
@@ -2054,6 +2080,8 @@ __global__ __launch_bounds__(kBlock) void k_injury_elem(InjuryArgs a) {
     a.flags[e] = fl;
     a.ps_old[e] = P[0];
     a.psxsr[e] = psxsr;
+    atomicAdd(&h[0][order_key(P[0]) >> sel_shift(0)], 1u);
+    atomicAdd(&h[1][order_key(psxsr) >> sel_shift(0)], 1u);
     bmax = {P[0], id};
     bmin = {P[1], id};
     bsh = {P[2], id};
@@ -2068,12 +2096,17 @@ __global__ __launch_bounds__(kBlock) void k_injury_elem(InjuryArgs a) {
     p[0] = bmax.v, p[1] = bmax.id, p[2] = bmin.v, p[3] = bmin.id;
     p[4] = bsh.v, p[5] = bsh.id, p[6] = bx.v, p[7] = bx.id;
   }
+  // (block_argbest's barriers lie between the counts and here)
+  for (int i = threadIdx.x; i < 2 * sel_bins(0); i += blockDim.x)
+    if ((&h[0][0])[i]) atomicAdd(&a.hist[sel_base(0) + i], (&h[0][0])[i]);
+  // the last pass's counters are cleared here, the others by k_injury_members
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 2 * sel_bins(kSelPasses - 1); i += gridDim.x * blockDim.x)
+    a.hist[sel_base(kSelPasses - 1) + i] = 0;
 }
 
 // The step's extrema over all blocks (block order, smallest id on ties), then
-// the running maxima with strict comparisons (ex5.cpp:1318-1366).
-__global__ __launch_bounds__(kBlock) void k_injury_reduce(InjuryArgs a, int nblk) {
-  if (a.slot && a.slot->done) return;
+// the running maxima with strict comparisons (ex5.cpp:1318-1366); one block.
+__device__ inline void injury_extrema(const InjuryArgs &a, int nblk) {
   const double ninf = -INFINITY;
   ArgBest r[4] = {{ninf, INT32_MAX}, {ninf, INT32_MAX}, {ninf, INT32_MAX}, {ninf, INT32_MAX}};
   for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
@@ -2095,96 +2128,132 @@ __global__ __launch_bounds__(kBlock) void k_injury_reduce(InjuryArgs a, int nblk
 }
 
 // 95th percentile (math.cpp:160-196 on one rank: the element at index
-// (int)(0.95 n) - 1 of the ascending order) of ps_old and of psxsr by a
-// radix select over order-preserving 64-bit keys, 8 bits per pass, both
-// arrays in the same launches.  sel[m]: {prefix, remaining rank}.
-__device__ inline unsigned long long order_key(double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
-}
-__device__ inline double key_value(unsigned long long k) {
-  const unsigned long long b = (k >> 63) ? (k & 0x7FFFFFFFFFFFFFFFull) : ~k;
-  return __longlong_as_double((long long)b);
-}
+// (int)(0.95 n) - 1 of the ascending order) of ps_old and of psxsr by a radix
+// select over order-preserving 64-bit keys, both arrays in the same launches:
+// 9 bits counted by k_injury_elem, then 5 x 11 bits.  Every block of the next
+// launch picks the digit from the finished histogram itself, so a digit costs
+// one launch; the last one is picked by k_injury_members.  Launch-bound on
+// meshes up to some 100,000 elements: with 8-bit digits, each picked by a
+// launch of one thread per array, an update took 21 launches and 197 us on
+// 33k elements; these 7 take 52 us (4 x 13 bits: 123 us, the larger
+// histograms cost more than the launch they save).
+//
+// sel[4 p + 2 m]: prefix and remaining rank of array m before pass p's digit
+// is picked.
+constexpr int kSelPer = (1 << kSelBits) / kBlock;  // bins per thread, at most
+struct SelPick {
+  unsigned long long key[2], rank[2];
+};
 
-__global__ void k_select_init(unsigned long long *sel, unsigned *hist, long n_incl, const StepSlot *slot) {
-  if (slot && slot->done) return;
-  long k = (long)(n_incl * 0.95) - 1;
-  if (k < 0) k = 0;
-  if (threadIdx.x < 2) {
-    sel[2 * threadIdx.x] = 0;
-    sel[2 * threadIdx.x + 1] = (unsigned long long)k;
-  }
-  for (int i = threadIdx.x; i < 512; i += blockDim.x) hist[i] = 0;
-}
-
-__global__ __launch_bounds__(kBlock) void k_select_hist(int ne, const int *flags, const double *v0,
-                                                        const double *v1, const unsigned long long *sel,
-                                                        int pass, unsigned *hist, const StepSlot *slot) {
-  if (slot && slot->done) return;
-  __shared__ unsigned h[2][256];
-  for (int i = threadIdx.x; i < 512; i += blockDim.x) h[i >> 8][i & 255] = 0;
-  __syncthreads();
-  const int shift = 56 - 8 * pass;
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += gridDim.x * blockDim.x) {
-    if (!(flags[e] & kInjIncluded)) continue;
-    const unsigned long long k0 = order_key(v0[e]), k1 = order_key(v1[e]);
-    if (pass == 0 || (k0 >> (shift + 8)) == sel[0]) atomicAdd(&h[0][(k0 >> shift) & 255], 1u);
-    if (pass == 0 || (k1 >> (shift + 8)) == sel[2]) atomicAdd(&h[1][(k1 >> shift) & 255], 1u);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < 512; i += blockDim.x)
-    if (h[i >> 8][i & 255]) atomicAdd(&hist[i], h[i >> 8][i & 255]);
-}
-
-// Picks the digit holding the remaining rank, extends the prefix, clears the
-// histogram for the next pass.
-__global__ void k_select_pick(unsigned long long *sel, unsigned *hist, const StepSlot *slot) {
-  if (slot && slot->done) return;
-  if (threadIdx.x < 2) {
-    const int m = threadIdx.x;
-    unsigned long long k = sel[2 * m + 1], cum = 0;
-    int b = 0;
-    for (; b < 255; ++b) {
-      if (k < cum + hist[256 * m + b]) break;
-      cum += hist[256 * m + b];
+// Prefix and remaining rank of both arrays after the digit of `pass`, in
+// every thread of a block of kBlock.
+__device__ inline SelPick select_pick(const unsigned *hist, const unsigned long long *sel, int pass, long n_incl) {
+  __shared__ unsigned long long sh_k[2], sh_r[2];
+  __shared__ unsigned sh_w[kBlock / 64];
+  const int bins = sel_bins(pass), per = bins / kBlock;
+  for (int m = 0; m < 2; ++m) {
+    unsigned long long prefix = 0, rank;
+    if (pass == 0) {
+      long k = (long)(n_incl * 0.95) - 1;
+      rank = (unsigned long long)(k < 0 ? 0 : k);
+    } else {
+      prefix = sel[4 * pass + 2 * m];
+      rank = sel[4 * pass + 2 * m + 1];
     }
-    sel[2 * m] = (sel[2 * m] << 8) | (unsigned long long)b;
-    sel[2 * m + 1] = k - cum;
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < 512; i += blockDim.x) hist[i] = 0;
-}
-
-// MPS-95 / MPSxSR-95 running maxima (ex5.cpp:1370-1429).
-__global__ void k_injury_p95(const unsigned long long *sel, double *scal, const StepSlot *slot, double time) {
-  if (slot && slot->done) return;
-  if (threadIdx.x < 2) {
-    const int m = threadIdx.x;
-    const double v = key_value(sel[2 * m]);
-    const double t = slot ? slot->t : time;
-    double *s = scal + 12 + 2 * m;
-    scal[16 + m] = 0.0;
-    if (v > s[0]) {
-      s[0] = v;
-      s[1] = t;
-      scal[16 + m] = 1.0;
+    const uint2 *h2 = reinterpret_cast<const uint2 *>(hist + sel_base(pass) + m * bins + threadIdx.x * per);
+    unsigned h[kSelPer], sum = 0;
+#pragma unroll
+    for (int i = 0; i < kSelPer / 2; ++i) {
+      const uint2 v = 2 * i < per ? h2[i] : make_uint2(0, 0);
+      h[2 * i] = v.x;
+      h[2 * i + 1] = v.y;
+      sum += v.x + v.y;
+    }
+    // exclusive prefix over the block's threads
+    unsigned inc = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+      const unsigned v = __shfl_up(inc, o);
+      if ((int)(threadIdx.x & 63) >= o) inc += v;
+    }
+    __syncthreads();  // the previous array's results have been read
+    if ((threadIdx.x & 63) == 63) sh_w[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    unsigned long long before = inc - sum;
+    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) before += sh_w[w];
+    // the thread whose bins hold the rank; the last bin when none does (an
+    // empty selection)
+    const bool mine = rank >= before && rank < before + sum;
+    if (mine || threadIdx.x == kBlock - 1) {
+      unsigned long long cum = before;
+      int b = 0;
+      bool found = false;
+#pragma unroll
+      for (int i = 0; i < kSelPer; ++i) {
+        found = found || i >= per - 1 || rank < cum + h[i];
+        if (!found) {
+          cum += h[i];
+          b = i + 1;
+        }
+      }
+      if (mine || rank >= before + sum) {
+        sh_k[m] = (prefix << (pass == 0 ? kSelFirst : kSelBits)) | (unsigned)(threadIdx.x * per + b);
+        sh_r[m] = rank - cum;
+      }
     }
   }
+  __syncthreads();
+  return {{sh_k[0], sh_k[1]}, {sh_r[0], sh_r[1]}};
 }
 
-// Element lists of a new MPS-95 / MPSxSR-95 maximum: value >= the maximum.
-__global__ __launch_bounds__(kBlock) void k_injury_members(int ne, int *flags, const double *ps_old,
-                                                           const double *psxsr, const double *scal,
-                                                           const StepSlot *slot) {
-  if (slot && slot->done) return;
+// Histogram of the digit of `pass` (>= 1) of the elements whose higher bits
+// are the prefix so far.  The first of these launches also reduces the
+// extrema and keeps the percentile maxima before this update.
+__global__ __launch_bounds__(kBlock) void k_select_hist(InjuryArgs a, unsigned long long *sel, int pass, long n_incl,
+                                                        int nblk) {
+  if (a.slot && a.slot->done) return;
+  __shared__ unsigned h[2][sel_bins(1)];
+  for (int i = threadIdx.x; i < 2 * sel_bins(1); i += blockDim.x) (&h[0][0])[i] = 0;
+  const SelPick p = select_pick(a.hist, sel, pass - 1, n_incl);  // (its barriers order the zeros)
+  if (blockIdx.x == 0 && threadIdx.x < 2) {
+    sel[4 * pass + 2 * threadIdx.x] = p.key[threadIdx.x];
+    sel[4 * pass + 2 * threadIdx.x + 1] = p.rank[threadIdx.x];
+  }
+  const int shift = sel_shift(pass);
+  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < a.ne; e += gridDim.x * blockDim.x) {
+    if (!(a.flags[e] & kInjIncluded)) continue;
+    const unsigned long long k0 = order_key(a.ps_old[e]), k1 = order_key(a.psxsr[e]);
+    if ((k0 >> (shift + kSelBits)) == p.key[0]) atomicAdd(&h[0][(k0 >> shift) & (sel_bins(1) - 1)], 1u);
+    if ((k1 >> (shift + kSelBits)) == p.key[1]) atomicAdd(&h[1][(k1 >> shift) & (sel_bins(1) - 1)], 1u);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 2 * sel_bins(1); i += blockDim.x)
+    if ((&h[0][0])[i]) atomicAdd(&a.hist[sel_base(pass) + i], (&h[0][0])[i]);
+  if (pass == 1 && blockIdx.x == 0) {
+    injury_extrema(a, nblk);
+    if (threadIdx.x < 2) a.scal[kInjOld + threadIdx.x] = a.scal[12 + 2 * threadIdx.x];
+  }
+}
+
+// MPS-95 / MPSxSR-95 running maxima (ex5.cpp:1370-1429) and the element lists
+// of a new one: value >= the maximum.  Clears the counters of the passes but
+// the last (which every block reads here).
+__global__ __launch_bounds__(kBlock) void k_injury_members(InjuryArgs a, const unsigned long long *sel, long n_incl) {
+  if (a.slot && a.slot->done) return;
+  const SelPick p = select_pick(a.hist, sel, kSelPasses - 1, n_incl);
+  const double v[2] = {key_value(p.key[0]), key_value(p.key[1])};
+  const bool up[2] = {v[0] > a.scal[kInjOld], v[1] > a.scal[kInjOld + 1]};
+  if (blockIdx.x == 0 && threadIdx.x < 2 && up[threadIdx.x]) {
+    a.scal[12 + 2 * threadIdx.x] = v[threadIdx.x];
+    a.scal[13 + 2 * threadIdx.x] = a.slot ? a.slot->t : a.time;
+  }
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < sel_base(kSelPasses - 1); i += gridDim.x * blockDim.x)
+    a.hist[i] = 0;
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
-  int fl = flags[e];
-  if (scal[16] != 0.0) fl = (fl & ~kInjMps95) | ((fl & kInjIncluded) && ps_old[e] >= scal[12] ? kInjMps95 : 0);
-  if (scal[17] != 0.0)
-    fl = (fl & ~kInjMpsxsr95) | ((fl & kInjIncluded) && psxsr[e] >= scal[14] ? kInjMpsxsr95 : 0);
-  flags[e] = fl;
+  if (e >= a.ne || !(up[0] || up[1])) return;
+  int fl = a.flags[e];
+  if (up[0]) fl = (fl & ~kInjMps95) | ((fl & kInjIncluded) && a.ps_old[e] >= v[0] ? kInjMps95 : 0);
+  if (up[1]) fl = (fl & ~kInjMpsxsr95) | ((fl & kInjIncluded) && a.psxsr[e] >= v[1] ? kInjMpsxsr95 : 0);
+  a.flags[e] = fl;
 }
 
 // Reference-configuration element volumes (calculateVolume,
@@ -3247,6 +3316,7 @@ InjuryArgs injury_args(ft_engine *g, const StepSlot *slot, double time, double d
   a.psxsr = g->inj_psxsr;
   a.part = g->inj_part;
   a.scal = g->inj_scal;
+  a.hist = g->inj_hist;
   a.slot = slot;
   a.time = time;
   a.dt = dt;
@@ -3260,17 +3330,10 @@ int injury_launch(ft_engine *g, const StepSlot *slot, double time, double dt) {
   const int nblk = (g->ne + kBlock - 1) / kBlock;
   const InjuryArgs a = injury_args(g, slot, time, dt);
   hipLaunchKernelGGL(k_injury_elem, dim3(nblk), dim3(kBlock), 0, g->stream, a);
-  hipLaunchKernelGGL(k_injury_reduce, dim3(1), dim3(kBlock), 0, g->stream, a, nblk);
-  hipLaunchKernelGGL(k_select_init, dim3(1), dim3(kBlock), 0, g->stream, g->inj_sel, g->inj_hist, g->inj_n, slot);
   const int sgrid = std::min(nblk, 1024);
-  for (int pass = 0; pass < 8; ++pass) {
-    hipLaunchKernelGGL(k_select_hist, dim3(sgrid), dim3(kBlock), 0, g->stream, g->ne, g->inj_flags, g->inj_ps_old,
-                       g->inj_psxsr, g->inj_sel, pass, g->inj_hist, slot);
-    hipLaunchKernelGGL(k_select_pick, dim3(1), dim3(kBlock), 0, g->stream, g->inj_sel, g->inj_hist, slot);
-  }
-  hipLaunchKernelGGL(k_injury_p95, dim3(1), dim3(64), 0, g->stream, g->inj_sel, g->inj_scal, slot, time);
-  hipLaunchKernelGGL(k_injury_members, dim3(nblk), dim3(kBlock), 0, g->stream, g->ne, g->inj_flags, g->inj_ps_old,
-                     g->inj_psxsr, g->inj_scal, slot);
+  for (int pass = 1; pass < kSelPasses; ++pass)
+    hipLaunchKernelGGL(k_select_hist, dim3(sgrid), dim3(kBlock), 0, g->stream, a, g->inj_sel, pass, g->inj_n, nblk);
+  hipLaunchKernelGGL(k_injury_members, dim3(nblk), dim3(kBlock), 0, g->stream, a, g->inj_sel, g->inj_n);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -5304,7 +5367,7 @@ int ft_injury_enable(ft_engine *g, const int *include_part) {
         (rc = dalloc(&g->inj_psxsr, ne)) || (rc = dalloc(&g->inj_vol, ne)) ||
         (rc = dalloc(&g->inj_part, 8 * (size_t)nblk)) || (rc = dalloc(&g->inj_scal, kInjScal)) ||
         (rc = dalloc(&g->inj_vpart, 5 * (size_t)nblk)) || (rc = dalloc(&g->inj_vsum, 5)) ||
-        (rc = dalloc(&g->inj_sel, 4)) || (rc = dalloc(&g->inj_hist, 512)))
+        (rc = dalloc(&g->inj_sel, 4 * kSelPasses)) || (rc = dalloc(&g->inj_hist, sel_base(kSelPasses))))
       return rc;
   }
   // included elements: parts with include_part[p] != 0 (ex5.cpp:1262-1281)
@@ -5324,6 +5387,7 @@ int ft_injury_enable(ft_engine *g, const int *include_part) {
   HIPCHK(hipMemcpy(g->inj_perm, g->perm.data(), ne * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK(hipMemset(g->inj_ps_old, 0, ne * sizeof(double)));  // ex5 leaves PS_Old unset; 0 here
   HIPCHK(hipMemset(g->inj_psxsr, 0, ne * sizeof(double)));
+  HIPCHK(hipMemset(g->inj_hist, 0, sel_base(kSelPasses) * sizeof(unsigned)));
   double sc[kInjScal];
   for (int k = 0; k < kInjScal; ++k) sc[k] = 0.0;
   sc[1] = sc[4] = sc[7] = sc[10] = -1.0;  // no element yet
