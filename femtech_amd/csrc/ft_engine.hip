@@ -2449,7 +2449,45 @@ __global__ void k_elem_flags(int ne, const int *conn, const unsigned char *node_
   einfo[e] = all ? (v | kSkipBit) : v;
 }
 
-// Velocity / acceleration read-out for ft_get_state.
+// Component-major [3][nn] to node-major [nn][3], and back.
+__global__ void k_to_node_major(int nn, const double *soa, double *aos) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= nn) return;
+  aos[3 * (size_t)n] = soa[n];
+  aos[3 * (size_t)n + 1] = soa[(size_t)nn + n];
+  aos[3 * (size_t)n + 2] = soa[2 * (size_t)nn + n];
+}
+__global__ void k_to_component_major(int nn, const double *aos, double *soa) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= nn) return;
+  soa[n] = aos[3 * (size_t)n];
+  soa[(size_t)nn + n] = aos[3 * (size_t)n + 1];
+  soa[2 * (size_t)nn + n] = aos[3 * (size_t)n + 2];
+}
+
+// Boundary motions at t = 0 (ex9.cpp:84) on the constrained DOFs of u and v.
+__global__ void k_motion_start(int nn, const int4 *tiles, int n_tiles, const double *X, const int *node_code,
+                               const double *motions, const int *mrange, double *u, double *v) {
+  const int L = blockIdx.x;
+  if (L >= n_tiles) return;
+  const int4 tile = tiles[L];
+  const int n = tile.x + threadIdx.x;
+  if (n >= tile.y) return;
+  const int code = node_code[n];
+  if (!code) return;
+  const double *mo = motions + (size_t)FT_MOTION_STRIDE * mrange[2 * tile.z];
+  const double Xn[3] = {X[n], X[(size_t)nn + n], X[2 * (size_t)nn + n]};
+  for (int d = 0; d < 3; ++d) {
+    const int mi = ((code >> (8 * d)) & 0xff) - 1;
+    if (mi < 0) continue;
+    double ub[3], vb[3], ab[3];
+    motion_eval(mo + FT_MOTION_STRIDE * mi, Xn, 0.0, ub, vb, ab);
+    u[(size_t)d * nn + n] = ub[d];
+    v[(size_t)d * nn + n] = vb[d];
+  }
+}
+
+// Acceleration read-out for ft_get_state (node-major).
 __global__ void k_state_out(int nn, const int4 *tiles, int n_tiles, const Ctl *ctl, int parity,
                             const double *fi, const double *mass, const double *X, const int *node_code,
                             const double *motions, const int *mrange, double *a_out) {
@@ -2464,12 +2502,12 @@ __global__ void k_state_out(int nn, const int4 *tiles, int n_tiles, const Ctl *c
     const int mi = ((node_code[n] >> (8 * d)) & 0xff) - 1;
     const size_t id = (size_t)d * nn + n;
     if (mi < 0) {
-      a_out[id] = (0.0 - fi[id]) / mass[n];
+      a_out[3 * (size_t)n + d] = (0.0 - fi[id]) / mass[n];
     } else {
       double ub[3], vb[3], ab[3];
       const double Xn[3] = {X[n], X[(size_t)nn + n], X[2 * (size_t)nn + n]};
       motion_eval(mo + FT_MOTION_STRIDE * mi, Xn, t, ub, vb, ab);
-      a_out[id] = ab[d];
+      a_out[3 * (size_t)n + d] = ab[d];
     }
   }
 }
@@ -2658,6 +2696,7 @@ struct ft_engine {
   unsigned long long *inj_sel = nullptr;
   unsigned *inj_hist = nullptr;
   // staging for the entry points that take host arrays every call
+  double *pin = nullptr;  // pinned, kPinnedBytes (allocated at first use)
   double *aux = nullptr;
   size_t aux_len = 0;
   double *scratch = nullptr;  // this device's copy of `scratch` (scratch_address)
@@ -2783,28 +2822,82 @@ void drop_graphs(ft_engine *g) {
 }
 
 // The device keeps nodal arrays component-major ([3][nn]); the C ABI uses the
-// reference's node-major layout (x[3 n + d]).
-std::vector<double> to_soa(const double *aos, size_t nn) {
-  std::vector<double> soa(3 * nn);
-  for (size_t n = 0; n < nn; ++n)
-    for (int d = 0; d < 3; ++d) soa[d * nn + n] = aos[3 * n + d];
-  return soa;
+// reference's node-major layout (x[3 n + d]).  Beyond kHostTranspose nodes the
+// caller's array goes to or comes from g->tmp3 as it is and the device
+// transposes; on the host the transposition and its fresh buffer took several
+// times the copy (2.0M nodes: ft_set_state of one array 28.2 -> 6.2 ms,
+// ft_get_state of four 63.6 -> 20.6 ms).  Up to kPinnedNodes nodes the copy
+// goes through the engine's pinned buffer: pinning the caller's pages for each
+// copy took longer than the copy (9,261 nodes, ft_get_state: 484 -> 134 us,
+// 121 us with the host's transposition).
+constexpr int kHostTranspose = 16384;
+constexpr int kPinnedNodes = 43690;
+constexpr size_t kPinnedBytes = 1 << 20;
+static_assert(3 * sizeof(double) * kPinnedNodes <= kPinnedBytes, "pinned buffer");
+
+int pinned(ft_engine *g, double **p) {
+  if (!g->pin && hipHostMalloc((void **)&g->pin, kPinnedBytes) != hipSuccess)
+    return fail(FT_ERR_ALLOC, "pinned buffer allocation failed");
+  *p = g->pin;
+  return 0;
 }
 
 int h2d_nodal(ft_engine *g, double *dev, const double *aos) {
-  std::vector<double> soa = to_soa(aos, g->nn);
-  HIPCHK(hipMemcpyAsync(dev, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));
+  const size_t nn = g->nn, bytes = 3 * nn * sizeof(double);
+  double *p = nullptr;
+  int rc;
+  if (g->nn <= kPinnedNodes && (rc = pinned(g, &p))) return rc;
+  if (g->nn <= kHostTranspose) {
+    for (size_t n = 0; n < nn; ++n)
+      for (int d = 0; d < 3; ++d) p[d * nn + n] = aos[3 * n + d];
+    HIPCHK(hipMemcpyAsync(dev, p, bytes, hipMemcpyHostToDevice, g->stream));
+  } else {
+    if (p) memcpy(p, aos, bytes);
+    HIPCHK(hipMemcpyAsync(g->tmp3, p ? p : aos, bytes, hipMemcpyHostToDevice, g->stream));
+    hipLaunchKernelGGL(k_to_component_major, dim3((g->nn + 255) / 256), dim3(256), 0, g->stream, g->nn, g->tmp3, dev);
+    HIPCHK(hipGetLastError());
+  }
   HIPCHK(hipStreamSynchronize(g->stream));
+  return 0;
+}
+
+// A node-major device array to the caller's (synchronises).
+int d2h_node_major(ft_engine *g, double *aos, const double *dev) {
+  const size_t bytes = 3 * (size_t)g->nn * sizeof(double);
+  double *p = nullptr;
+  int rc;
+  if (g->nn <= kPinnedNodes && (rc = pinned(g, &p))) return rc;
+  HIPCHK(hipMemcpyAsync(p ? p : aos, dev, bytes, hipMemcpyDeviceToHost, g->stream));
+  HIPCHK(hipStreamSynchronize(g->stream));
+  if (p) memcpy(aos, p, bytes);
   return 0;
 }
 
 int d2h_nodal(ft_engine *g, double *aos, const double *dev) {
   const size_t nn = g->nn;
-  std::vector<double> soa(3 * nn);
-  HIPCHK(hipMemcpyAsync(soa.data(), dev, soa.size() * sizeof(double), hipMemcpyDeviceToHost, g->stream));
+  if (g->nn <= kHostTranspose) {
+    double *p = nullptr;
+    int rc;
+    if ((rc = pinned(g, &p))) return rc;
+    HIPCHK(hipMemcpyAsync(p, dev, 3 * nn * sizeof(double), hipMemcpyDeviceToHost, g->stream));
+    HIPCHK(hipStreamSynchronize(g->stream));
+    for (size_t n = 0; n < nn; ++n)
+      for (int d = 0; d < 3; ++d) aos[3 * n + d] = p[d * nn + n];
+    return 0;
+  }
+  hipLaunchKernelGGL(k_to_node_major, dim3((g->nn + 255) / 256), dim3(256), 0, g->stream, g->nn, dev, g->tmp3);
+  HIPCHK(hipGetLastError());
+  return d2h_node_major(g, aos, g->tmp3);
+}
+
+// A few values to the host, behind the stream's work (synchronises).
+int d2h_small(ft_engine *g, void *dst, const void *src, size_t bytes) {
+  double *p = nullptr;
+  int rc;
+  if (bytes <= kPinnedBytes && (rc = pinned(g, &p))) return rc;
+  HIPCHK(hipMemcpyAsync(p ? (void *)p : dst, src, bytes, hipMemcpyDeviceToHost, g->stream));
   HIPCHK(hipStreamSynchronize(g->stream));
-  for (size_t n = 0; n < nn; ++n)
-    for (int d = 0; d < 3; ++d) aos[3 * n + d] = soa[d * nn + n];
+  if (p) memcpy(dst, p, bytes);
   return 0;
 }
 
@@ -3711,8 +3804,8 @@ int upload_caps(ft_engine *g, const std::vector<int> &cap) {
 
 int read_slots(ft_engine *g, int parity, std::vector<StepSlot> &s) {
   std::vector<Ctl> c(g->n_inst);
-  HIPCHK(hipMemcpyAsync(c.data(), g->ctl, c.size() * sizeof(Ctl), hipMemcpyDeviceToHost, g->stream));
-  HIPCHK(hipStreamSynchronize(g->stream));
+  int rc = d2h_small(g, c.data(), g->ctl, c.size() * sizeof(Ctl));
+  if (rc) return rc;
   s.resize(g->n_inst);
   for (int i = 0; i < g->n_inst; ++i) s[i] = c[i].slot[parity];
   return 0;
@@ -3737,17 +3830,14 @@ int aux_reserve(ft_engine *g, size_t len) {
 }
 
 int check_status(ft_engine *g) {
-  int st = 0;
-  HIPCHK(hipMemcpyAsync(&st, g->status, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-  HIPCHK(hipStreamSynchronize(g->stream));
+  int st = 0, rc;
+  if ((rc = d2h_small(g, &st, g->status, sizeof(int)))) return rc;
   if (st & 8) return fail(FT_ERR_MATERIAL, "unknown material type");
   return 0;
 }
 
 int read_slot(ft_engine *g, int parity, StepSlot *s) {
-  HIPCHK(hipMemcpyAsync(s, &g->ctl->slot[parity], sizeof(StepSlot), hipMemcpyDeviceToHost, g->stream));
-  HIPCHK(hipStreamSynchronize(g->stream));
-  return 0;
+  return d2h_small(g, s, &g->ctl->slot[parity], sizeof(StepSlot));
 }
 
 }  // namespace
@@ -3980,10 +4070,7 @@ int ft_engine_create(int n_nodes, int n_elems, const double *coords, const int *
     hinfo[i] = pid[e];
     for (int k = 0; k < 8; ++k) hconn[8 * (size_t)i + k] = conn[8 * (size_t)e + k];
   }
-  {
-    std::vector<double> soa = to_soa(coords, n_nodes);
-    HIPCHK_BAIL(hipMemcpy(g->X, soa.data(), nd * sizeof(double), hipMemcpyHostToDevice));
-  }
+  if ((rc = h2d_nodal(g, g->X, coords))) return bail(rc);
   HIPCHK_BAIL(hipMemcpy(g->conn, hconn.data(), 8 * (size_t)n_elems * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK_BAIL(hipMemcpy(g->einfo, hinfo.data(), (size_t)n_elems * sizeof(int), hipMemcpyHostToDevice));
   HIPCHK_BAIL(hipMemcpy(g->parts, g->h_parts.data(), n_parts * sizeof(PartDev), hipMemcpyHostToDevice));
@@ -4039,6 +4126,7 @@ int ft_engine_destroy(ft_engine *g) {
   for (void *p : {(void *)g->snap_dev, (void *)g->snap_ctl_dev})
     if (p) (void)hipFree(p);
   if (g->h_ctl) (void)hipHostFree(g->h_ctl);
+  if (g->pin) (void)hipHostFree(g->pin);
   if (g->stream) (void)hipStreamDestroy(g->stream);
   delete g;
   return 0;
@@ -4191,8 +4279,7 @@ int ft_stable_time_step(ft_engine *g, const double *u, const int *boundary, doub
   std::vector<unsigned long long> bits(g->n_inst, kInfBits);
   HIPCHK(hipMemcpyAsync(g->dtbits, bits.data(), bits.size() * sizeof(bits[0]), hipMemcpyHostToDevice, g->stream));
   if ((rc = element_pass(g, false, true, false, 0.0, g->dtbits, 0))) return rc;
-  HIPCHK(hipMemcpyAsync(bits.data(), g->dtbits, bits.size() * sizeof(bits[0]), hipMemcpyDeviceToHost, g->stream));
-  HIPCHK(hipStreamSynchronize(g->stream));
+  if ((rc = d2h_small(g, bits.data(), g->dtbits, bits.size() * sizeof(bits[0])))) return rc;
   const unsigned long long bmin = *std::min_element(bits.begin(), bits.end());
   double dt;
   memcpy(&dt, &bmin, sizeof(dt));
@@ -4338,24 +4425,11 @@ int ft_run_init(ft_engine *g, double tmax, double dt_factor, double failure_dt) 
   g->failure_dt = failure_dt;
   g->parity = 0;
   g->run_active = false;
-  // Boundary motions at t = 0 (ex9.cpp:84) on the constrained DOFs.
-  const size_t nd = 3 * (size_t)g->nn;
   if (g->n_motions > 0) {
-    std::vector<double> X(nd), u(nd), v(nd);
-    int rc;
-    if ((rc = d2h_nodal(g, X.data(), g->X)) || (rc = d2h_nodal(g, u.data(), g->u)) ||
-        (rc = d2h_nodal(g, v.data(), g->vs)))
-      return rc;
-    for (int n = 0; n < g->nn; ++n)
-      for (int d = 0; d < 3; ++d) {
-        int mi = g->h_dof_motion[3 * n + d];
-        if (mi < 0) continue;
-        double ub[3], vb[3], ab[3];
-        motion_eval(&g->h_motions[FT_MOTION_STRIDE * mi], &X[3 * n], 0.0, ub, vb, ab);
-        u[3 * n + d] = ub[d];
-        v[3 * n + d] = vb[d];
-      }
-    if ((rc = h2d_nodal(g, g->u, u.data())) || (rc = h2d_nodal(g, g->vs, v.data()))) return rc;
+    hipLaunchKernelGGL(k_motion_start, dim3(std::max(1, g->n_ntiles)), dim3(kBlock), 0, g->stream, g->nn, g->ntiles,
+                       g->n_ntiles, g->X, g->node_code, g->motions, g->mrange, g->u, g->vs);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(g->stream));  // the copies below do not wait for the engine's stream
   }
   HIPCHK(hipMemset(g->eacc, 0, kEaccStride * (size_t)std::max(1, g->n_ntiles) * sizeof(double)));
   HIPCHK(hipMemset(g->status, 0, sizeof(int)));
@@ -4539,7 +4613,7 @@ int ft_run_steps(ft_engine *g, int max_steps, int *steps_done) {
   for (int i = 0; i < g->n_inst; ++i) done = std::max(done, s[i].step - before[i]);
   if (steps_done) *steps_done = done;
   int st = 0;
-  HIPCHK(hipMemcpy(&st, g->status, sizeof(int), hipMemcpyDeviceToHost));
+  if ((rc = d2h_small(g, &st, g->status, sizeof(int)))) return rc;
   if (st & kStatusBarrier) return fail(FT_ERR_HIP, "persistent launch: a grid barrier wait ran out; the run is void");
   if (st & 8) return fail(FT_ERR_MATERIAL, "Unknown material type");
   // A batch keeps going when one of its instances stops without a stable
@@ -4564,15 +4638,6 @@ int ft_get_time(ft_engine *g, double *time, double *dt, int *step) {
   if (dt) *dt = g->run_active ? s.dt_done : 0.0;
   if (step) *step = s.step;
   return 0;
-}
-
-// Component-major [3][nn] to node-major [nn][3].
-__global__ void k_to_node_major(int nn, const double *soa, double *aos) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= nn) return;
-  aos[3 * (size_t)n] = soa[n];
-  aos[3 * (size_t)n + 1] = soa[(size_t)nn + n];
-  aos[3 * (size_t)n + 2] = soa[2 * (size_t)nn + n];
 }
 
 // A node-major copy of the current displacement (and the control slots) is
@@ -4636,20 +4701,16 @@ int ft_snapshot_end(ft_engine *g, double *u, double *time, int *step) {
 
 int ft_get_state(ft_engine *g, double *u, double *v, double *a, double *fi) {
   if (!g) return fail(FT_ERR_ARG, "null engine");
-  const size_t nb = 3 * (size_t)g->nn * sizeof(double);
-  HIPCHK(hipStreamSynchronize(g->stream));
-  (void)nb;
   int rc0;
   if (u && (rc0 = d2h_nodal(g, u, g->u))) return rc0;
   if (v && (rc0 = d2h_nodal(g, v, g->vs))) return rc0;
   if (fi && (rc0 = d2h_nodal(g, fi, g->fi))) return rc0;
   if (a) {
-    int rc;
     hipLaunchKernelGGL(k_state_out, dim3(std::max(1, g->n_ntiles)), dim3(kBlock), 0, g->stream, g->nn, g->ntiles,
                        g->n_ntiles, g->ctl, g->parity, g->fi, g->mass, g->X, g->node_code, g->motions, g->mrange,
                        g->tmp3);
     HIPCHK(hipGetLastError());
-    if ((rc = d2h_nodal(g, a, g->tmp3))) return rc;
+    if ((rc0 = d2h_node_major(g, a, g->tmp3))) return rc0;
   }
   return 0;
 }
