@@ -269,26 +269,27 @@ __device__ inline uint64_t mix64(uint64_t z) {
 // ---------------------------------------------------------------------------
 // Training
 // ---------------------------------------------------------------------------
-// k_mlp_train: one block takes 128 samples through forward, loss and backward:
-// 4 wavefronts of 32 samples each, one per SIMD, every product with W^T-shaped
-// A operands from LDS (rows padded by 16 bytes, as in k_mlp_infer) against the
-// wavefront's own samples as B operands, so activations and their gradients
-// pass from layer to layer in registers (the whole register file; SiLU' of the
-// first layer in LDS): an output tile's accumulators (lane half h: rows 8 j +
-// 4 h + r) become B operands (depth 8 h + i) by one v_permlane32_swap per
-// packed pair.  The barriers only guard the weights' two buffers.  For the
-// weight gradients, whose depth is the samples, activations and dZ go to
-// memory sample-contiguous; k_mlp_grad spreads their 56 tiles per 256 samples
-// over the chip.  Every sum keeps its order: products in steps of 16, weight
-// gradients in blocks of 256 samples added in order, bias gradients by 256
-// strided sums and a tree, so a step does not depend on how samples are
-// spread over blocks.
+// k_mlp_train: one block takes 32 samples through forward, loss and backward.
+// Its 4 wavefronts each own 32 of a layer's 128 rows: weights as A operands
+// straight from the cache into registers, a layer ahead, against the block's
+// samples as B operands.  A tile's accumulators (lane half h: rows 8 j + 4 h +
+// r) become B operands (depth 8 h + i) by one v_permlane32_swap per packed
+// pair and go to the other wavefronts through LDS, two buffers, one barrier per
+// layer; SiLU' stays in registers.  For the weight gradients, whose depth is
+// the samples, activations and dZ go to memory sample-contiguous; k_mlp_grad
+// spreads their 56 tiles per 256 samples over the chip.  Every sum keeps its
+// order: products in steps of 16, weight gradients in blocks of 256 samples
+// added in order, bias gradients by 256 strided sums and a tree, so a step does
+// not depend on how samples are spread over blocks.
 // A step is a chain of small products: bound by latency and by the SiLU
-// evaluations, not by the matrix cores.  As 37 launches of single products and
-// elementwise passes it took 540 us at a batch of 4,096; as three, 85 us
-// (64 + 15 + 5).
-constexpr int kTrainTile = 128;     // samples per block
-constexpr int kTrainThreads = 256;  // 4 wavefronts x 32 samples
+// evaluations, not by the matrix cores, so the rows are split, not only the
+// samples.  A step at a batch of 1,024 / 4,096 / 65,536: 28 / 40 / 295 us;
+// 59 / 82 / 378 us with 32 samples and all rows per wavefront (4 to a block,
+// weights staged in LDS, SiLU' spilled); 540 us at 4,096 as 37 launches of
+// single products and elementwise passes.  At 2 wavefronts per SIMD (44 bytes
+// of spills) instead of 1, 65,536 takes 295 instead of 323 us, 4,096 the same.
+constexpr int kTrainTile = 32;      // samples per block
+constexpr int kTrainThreads = 256;  // 4 wavefronts x 32 rows of a layer
 constexpr int kGradChunk = 256;     // samples per weight-gradient block
 constexpr int kAtRows = kMlpIn + 4 * kMlpHid, kDzRows = 4 * kMlpHid + kMlpOut;
 
@@ -304,7 +305,7 @@ struct TrainArgs {
   __bf16 *at;           // activations [input 16, layers 1-4 128 each][ld]; zero past n
   __bf16 *dzb;          // dZ of layers 0-4 (128, ..., 8 rows) [ld], BF16 and FP32; zero past n
   float *dz;
-  double *lpart;        // squared errors by block
+  double *lpart;        // squared errors by block of samples
 };
 
 // Accumulators of a 32-row tile (rows 8 j + 4 h + r) as the two B operands of
@@ -346,188 +347,132 @@ __device__ __forceinline__ void silu_both(float z, float &v, float &d) {
   d = s * (1.0f + z * (1.0f - s));
 }
 
-// The products of a layer: acc[t] = sum_k W(32 t + c32, 16 k + ..) B[k], weight
-// rows at `wl` (LDS, row stride kPadW).
+// Weights of this lane's row of a product (16 STEPS deep), as A operands.
 template <int STEPS>
-__device__ __forceinline__ void layer_product(const __bf16 *wl, int c32, int h, const bf16x8 (&B)[8], f32x16 (&acc)[4]) {
+__device__ __forceinline__ void fetch_row(const __bf16 *row, int h, bf16x8 (&A)[8]) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f32x16{};
-#pragma unroll
-  for (int k = 0; k < STEPS; ++k)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(wl + (32 * t + c32) * kPadW + 16 * k + 8 * h);
-      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[k], acc[t], 0, 0, 0);
-    }
+  for (int k = 0; k < STEPS; ++k) A[k] = *reinterpret_cast<const bf16x8 *>(row + 16 * k + 8 * h);
 }
 
-struct TrainLds {
-  __attribute__((aligned(16))) __bf16 w[2][kMlpHid * kPadW];  // weights of this layer and the next
-  float zg0[4][64][64];                                       // SiLU'(Z_0) by wavefront and lane
-  float b[kMlpLayers * kMlpHid];                              // biases
-  double loss[4];
-};
+template <int STEPS>
+__device__ __forceinline__ f32x16 row_product(const bf16x8 (&A)[8], const bf16x8 (&B)[8]) {
+  f32x16 acc = {};
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[k], B[k], acc, 0, 0, 0);
+  return acc;
+}
 
-__global__ __launch_bounds__(kTrainThreads) void k_mlp_train(TrainArgs g) {
-  __shared__ TrainLds lds;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, c32 = lane & 31;
-  const size_t i = (size_t)blockIdx.x * kTrainTile + 32 * w + c32;  // sample in the batch (below ld)
+__global__ __launch_bounds__(kTrainThreads, 2) void k_mlp_train(TrainArgs g) {
+  __shared__ bf16x8 ex[2][8][64];  // a layer's output as the next one's B operands, [32-row tile, half][lane]
+  const int lane = threadIdx.x & 63, h = lane >> 5, c32 = lane & 31;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int r0 = 32 * w + c32;                                // this lane's row of A in a product
+  const size_t i = (size_t)blockIdx.x * kTrainTile + c32;     // sample in the batch (below ld)
   const bool valid = i < (size_t)g.n;
   const bf16x8 zero8 = {};
-  // weights of a product: rows x 128 (or 16) deep, 16 bytes per thread and turn, through registers
-  constexpr int kTurns = kMlpHid * kMlpHid / 8 / kTrainThreads;
-  bf16x8 pre[kTurns];
-  auto fetch = [&](const __bf16 *src, int chunks) {
-#pragma unroll
-    for (int k = 0; k < kTurns; ++k) {
-      const int c = k * kTrainThreads + (int)threadIdx.x;
-      if (c < chunks) pre[k] = reinterpret_cast<const bf16x8 *>(src)[c];
-    }
-  };
-  auto stage = [&](int buf, int chunks, int per_row) {
-#pragma unroll
-    for (int k = 0; k < kTurns; ++k) {
-      const int c = k * kTrainThreads + (int)threadIdx.x;
-      if (c < chunks) *reinterpret_cast<bf16x8 *>(&lds.w[buf][(c / per_row) * kPadW + (c % per_row) * 8]) = pre[k];
-    }
-  };
-  constexpr int kFull = kMlpHid * kMlpHid / 8, kIn = kMlpHid * kMlpIn / 8, kOut = kMlpOut * kMlpHid / 8;
-  constexpr int kOutT = kMlpHid * 16 / 8;
-  fetch(g.Pb + w_off(0), kIn);
-  for (int k = threadIdx.x; k < kMlpLayers * kMlpHid; k += kTrainThreads) {
-    const int l = k / kMlpHid, r = k % kMlpHid;
-    lds.b[k] = r < layer_out(l) ? g.P[b_off(l) + r] : 0.0f;
-  }
+  bf16x8 A[2][8], B[8];  // weights of a layer and of the next
+  fetch_row<1>(g.Pb + w_off(0) + r0 * kMlpIn, h, A[0]);
   size_t row = i;
   if (g.n_data > 0) row = (size_t)(mix64(g.key ^ (uint64_t)i * 0xD1B54A32D192ED03ull) % (uint64_t)g.n_data);
-  bf16x8 B[8];
   B[0] = valid ? *reinterpret_cast<const bf16x8 *>(g.x + row * kMlpIn + 8 * h) : zero8;
   const float4 tv = valid ? *reinterpret_cast<const float4 *>(g.t + row * kMlpOut + 4 * h) : float4{0, 0, 0, 0};
+  if (w == 0) {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) g.at[(8 * h + k) * g.ld + i] = B[0][k];
-  stage(0, kIn, kMlpIn / 8);
-  fetch(g.Pb + w_off(1), kFull);
-  __syncthreads();
-  // ---- forward: Z_l = W_l A_{l-1} + b_l, A_l = SiLU(Z_l); layer l's weights are in buffer l % 2
-  float zg[3][64];  // SiLU'(Z_l), l = 1-3
-  f32x16 acc[4];
+    for (int k = 0; k < 8; ++k) g.at[(8 * h + k) * g.ld + i] = B[0][k];
+  }
+  // ---- forward: Z_l = W_l A_{l-1} + b_l, A_l = SiLU(Z_l)
+  float zg[4][16];  // SiLU'(Z_l), l = 0-3
 #pragma unroll
   for (int l = 0; l < 4; ++l) {
-    if (l == 0)
-      layer_product<1>(lds.w[0], c32, h, B, acc);
-    else
-      layer_product<8>(lds.w[l & 1], c32, h, B, acc);
-    __bf16 *al = g.at + (size_t)(kMlpIn + l * kMlpHid) * g.ld + i;
+    float4 b4[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float v[16];
+    for (int j = 0; j < 4; ++j) b4[j] = *reinterpret_cast<const float4 *>(g.P + b_off(l) + 32 * w + 8 * j + 4 * h);
+    if (l < 3) {
+      fetch_row<8>(g.Pb + w_off(l + 1) + r0 * kMlpHid, h, A[(l + 1) & 1]);
+    } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int f = 32 * t + 8 * j + 4 * h;
-        const float4 b4 = *reinterpret_cast<const float4 *>(&lds.b[l * kMlpHid + f]);
-        const float bb[4] = {b4.x, b4.y, b4.z, b4.w};
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int e = 4 * j + r;
-          float d;
-          silu_both(acc[t][e] + bb[r], v[e], d);
-          if (l == 0)
-            lds.zg0[w][16 * t + e][lane] = d;
-          else
-            zg[l - 1][16 * t + e] = d;
-          al[(size_t)(f + r) * g.ld] = valid ? (__bf16)v[e] : (__bf16)0.0f;
-        }
-      }
-      bf16x8 two[2];
-      tile_to_operands(v, two);
-      B[2 * t] = two[0];
-      B[2 * t + 1] = two[1];
+      for (int k = 0; k < 8; ++k) A[0][k] = zero8;
+      if (c32 < kMlpOut) fetch_row<8>(g.Pb + w_off(4) + c32 * kMlpHid, h, A[0]);
     }
-    // the next layer's weights into the other buffer (its last readers passed the barrier before)
-    if (l < 3)
-      stage((l + 1) & 1, kFull, kMlpHid / 8);
-    else
-      stage(0, kOut, kMlpHid / 8);
-    if (l < 2)
-      fetch(g.Pb + w_off(l + 2), kFull);
-    else if (l == 2)
-      fetch(g.Pb + w_off(4), kOut);
-    else
-      fetch(g.Wt + wt_off(4), kOutT);
-    __syncthreads();
-  }
-  // ---- output layer, loss: mean squared error over the 6 used outputs
-  f32x16 o = {};
+    const f32x16 acc = l == 0 ? row_product<1>(A[0], B) : row_product<8>(A[l & 1], B);
+    __bf16 *al = g.at + (size_t)(kMlpIn + l * kMlpHid + 32 * w) * g.ld + i;
+    float v[16];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const bf16x8 a =
-        c32 < kMlpOut ? *reinterpret_cast<const bf16x8 *>(&lds.w[0][c32 * kPadW + 16 * k + 8 * h]) : zero8;
-    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[k], o, 0, 0, 0);
+    for (int j = 0; j < 4; ++j) {
+      const float bb[4] = {b4[j].x, b4[j].y, b4[j].z, b4[j].w};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int e = 4 * j + r;
+        silu_both(acc[e] + bb[r], v[e], zg[l][e]);
+        al[(size_t)(8 * j + 4 * h + r) * g.ld] = valid ? (__bf16)v[e] : (__bf16)0.0f;
+      }
+    }
+    bf16x8 two[2];
+    tile_to_operands(v, two);
+    ex[l & 1][2 * w][lane] = two[0];
+    ex[l & 1][2 * w + 1][lane] = two[1];
+    __syncthreads();  // (buffer l & 1 is written again two layers on, past the next barrier)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) B[k] = ex[l & 1][k][lane];
   }
-  stage(1, kOutT, 2);  // W4^T (layer 3's weights were last read before the barrier)
-  fetch(g.Wt + wt_off(3), kFull);
+  // ---- output layer and loss, alike in every wavefront: mean squared error over the 6 used outputs
+  const float4 bo = *reinterpret_cast<const float4 *>(g.P + b_off(4) + 4 * h);
+  fetch_row<1>(g.Wt + wt_off(4) + r0 * 16, h, A[1]);
+  const f32x16 o = row_product<8>(A[0], B);
+  fetch_row<8>(g.Wt + wt_off(3) + r0 * kMlpHid, h, A[0]);
   float dy[4];
   double e2 = 0.0;
   {
-    const float tt[4] = {tv.x, tv.y, tv.z, tv.w};
+    const float tt[4] = {tv.x, tv.y, tv.z, tv.w}, bb[4] = {bo.x, bo.y, bo.z, bo.w};
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int k = 4 * h + r;
-      const float d = (o[r] + lds.b[4 * kMlpHid + k]) - tt[r];
+      const float d = (o[r] + bb[r]) - tt[r];
       const bool use = valid && k < kMlpUsedOut;
       dy[r] = use ? 2.0f * d / (float)(kMlpUsedOut * (long)g.n) : 0.0f;
       if (use) e2 += (double)d * d;
     }
   }
-  for (int m = 32; m > 0; m >>= 1) e2 += __shfl_xor(e2, m);
-  if (lane == 0) lds.loss[w] = e2;
   // dZ of the output layer: to memory, and as the B operand (depth 8: the lower half holds all 8)
   B[0] = zero8;
-  {
-    float other[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) other[r] = __shfl_xor(dy[r], 32);
+  for (int r = 0; r < 4; ++r) {
+    const float other = __shfl_xor(dy[r], 32);
+    B[0][r] = h ? (__bf16)0.0f : (__bf16)dy[r];
+    B[0][4 + r] = h ? (__bf16)0.0f : (__bf16)other;
+  }
+  if (w == 0) {
+    for (int m = 32; m > 0; m >>= 1) e2 += __shfl_xor(e2, m);
+    if (lane == 0) g.lpart[blockIdx.x] = e2;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      B[0][r] = h ? (__bf16)0.0f : (__bf16)dy[r];
-      B[0][4 + r] = h ? (__bf16)0.0f : (__bf16)other[r];
       const size_t at = (size_t)(4 * kMlpHid + 4 * h + r) * g.ld + i;
       g.dz[at] = dy[r];
       g.dzb[at] = (__bf16)dy[r];
     }
   }
-  __syncthreads();
-  if (threadIdx.x == 0) g.lpart[blockIdx.x] = lds.loss[0] + lds.loss[1] + lds.loss[2] + lds.loss[3];
-  // ---- backward: dA_{l-1} = W_l^T dZ_l (W_l^T in buffer (l + 1) % 2); dZ_{l-1} = dA SiLU'(Z_{l-1})
+  // ---- backward: dA_{l-1} = W_l^T dZ_l; dZ_{l-1} = dA SiLU'(Z_{l-1})
 #pragma unroll
   for (int l = 4; l >= 1; --l) {
-    if (l == 4)
-      layer_product<1>(lds.w[1], c32, h, B, acc);
-    else
-      layer_product<8>(lds.w[(l + 1) & 1], c32, h, B, acc);
+    const f32x16 acc = l == 4 ? row_product<1>(A[1], B) : row_product<8>(A[(l + 1) & 1], B);
+    if (l == 4 || l == 3) fetch_row<8>(g.Wt + wt_off(l - 2) + r0 * kMlpHid, h, A[(l + 1) & 1]);
+    float v[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const size_t at = (size_t)((l - 1) * kMlpHid + 32 * w + 8 * (e >> 2) + 4 * h + (e & 3)) * g.ld + i;
+      v[e] = valid ? acc[e] * zg[l - 1][e] : 0.0f;
+      g.dz[at] = v[e];
+      g.dzb[at] = (__bf16)v[e];
+    }
     if (l > 1) {
-      stage(l & 1, kFull, kMlpHid / 8);  // W_{l-1}^T
-      if (l > 2) fetch(g.Wt + wt_off(l - 2), kFull);
-    }
+      bf16x8 two[2];
+      tile_to_operands(v, two);
+      ex[l & 1][2 * w][lane] = two[0];
+      ex[l & 1][2 * w + 1][lane] = two[1];
+      __syncthreads();
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float v[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const size_t at = (size_t)((l - 1) * kMlpHid + 32 * t + 8 * (e >> 2) + 4 * h + (e & 3)) * g.ld + i;
-        const float d = l == 1 ? lds.zg0[w][16 * t + e][lane] : zg[l > 1 ? l - 2 : 0][16 * t + e];
-        v[e] = valid ? acc[t][e] * d : 0.0f;
-        g.dz[at] = v[e];
-        g.dzb[at] = (__bf16)v[e];
-      }
-      if (l > 1) {
-        bf16x8 two[2];
-        tile_to_operands(v, two);
-        B[2 * t] = two[0];
-        B[2 * t + 1] = two[1];
-      }
+      for (int k = 0; k < 8; ++k) B[k] = ex[l & 1][k][lane];
     }
-    if (l > 1) __syncthreads();
   }
 }
 
@@ -705,11 +650,11 @@ int train_batch(MlpNet *net, const __bf16 *x, const float *t, long n_data, uint6
 }
 
 int read_loss(MlpNet *net, int n, hipStream_t st, double *loss) {
-  std::vector<double> part(((size_t)n + kTrainTile - 1) / kTrainTile);
+  std::vector<double> part(train_ld(n) / kTrainTile);
   MCHK(hipMemcpyAsync(part.data(), net->lpart, part.size() * sizeof(double), hipMemcpyDeviceToHost, st));
   MCHK(hipStreamSynchronize(st));
   double s = 0.0;
-  for (double p : part) s += p;
+  for (size_t k = 0; k < part.size(); k += 4) s += part[k] + part[k + 1] + part[k + 2] + part[k + 3];
   *loss = s / ((double)n * kMlpUsedOut);
   return 0;
 }
