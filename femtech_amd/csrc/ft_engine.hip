@@ -1064,10 +1064,17 @@ __global__ __launch_bounds__(kBlock) void k_element_gp(ElemArgs<R> a) {
   element_tile<R, true, false, -1, false, true>(a, xcd_block());
 }
 
-// Run-loop element kernel of a surrogate segment (FP32, force + dt).
-template <int MAT>
+// Run-loop element kernel of the surrogate segments (FP32, force + dt), each
+// tile with its law's body (both take 2 wavefronts per SIMD).  One launch: by
+// itself a law with few elements takes the time of its longest chain (5,400
+// elements of material 8: 32 us beside 106 us for 165,000 of material 7).
 __global__ __launch_bounds__(kBlock) void k_element_surr(ElemArgs<float> a) {
-  element_tile<float, true, true, MAT, true>(a, xcd_block());
+  const int L = xcd_block();
+  if (L >= a.n_tiles) return;
+  if (a.tiles[L].w >> kTileMat == 7)  // uniform over the block
+    element_tile<float, true, true, 7, true>(a, L);
+  else
+    element_tile<float, true, true, 8, true>(a, L);
 }
 
 // grad_X u at Gauss point gp from the normalised coefficients of x and u
@@ -1171,17 +1178,12 @@ __global__ __launch_bounds__(kBlock) void k_surr_sample(int nn, int ne, const in
   }
 }
 
-// Network inputs of a surrogate segment's Gauss points at the run loop's
-// displacement (FP32, as the element kernel forms them), normalised, BF16,
-// Gauss-point major.
+// Network inputs of the surrogate segments' Gauss points (elements [e0, e8) of
+// material 7, [e8, e1) of material 8) at the run loop's displacement (FP32, as
+// the element kernel forms them), normalised, BF16, Gauss-point major.
 template <int MAT>
-__global__ __launch_bounds__(kBlock) void k_surr_features(int nn, int ne, const int *conn, const double *X,
-                                                          const double *u, const float *fibf, int e0, int e1,
-                                                          const float *norm, __bf16 *feat, const Ctl *ctl,
-                                                          int parity) {
-  const int e = e0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= e1) return;
-  if (ctl[0].slot[parity].done) return;
+__device__ inline void surr_features_of(int nn, int ne, const int *conn, const double *X, const double *u,
+                                        const float *fibf, int e0, int e1, int e, const float *norm, __bf16 *feat) {
   float cx[7][3], cu[7][3], fib[3];
   element_coeffs<float>(nn, ne, conn, X, u, fibf, nullptr, e, cx, cu, fib);
   float Q[3][3];
@@ -1197,6 +1199,19 @@ __global__ __launch_bounds__(kBlock) void k_surr_features(int nn, int ne, const 
 #pragma unroll
     for (int k = 0; k < kSurrFeat; ++k) dst[k] = (__bf16)((f[k] - norm[k]) / norm[16 + k]);
   }
+}
+
+__global__ __launch_bounds__(kBlock) void k_surr_features(int nn, int ne, const int *conn, const double *X,
+                                                          const double *u, const float *fibf, int e0, int e8, int e1,
+                                                          const float *norm, __bf16 *feat, const Ctl *ctl,
+                                                          int parity) {
+  const int e = e0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= e1) return;
+  if (ctl[0].slot[parity].done) return;
+  if (e < e8)
+    surr_features_of<7>(nn, ne, conn, X, u, fibf, e0, e1, e, norm, feat);
+  else
+    surr_features_of<8>(nn, ne, conn, X, u, fibf, e0, e1, e, norm, feat);
 }
 
 // ---------------------------------------------------------------------------
@@ -3173,59 +3188,55 @@ int element_pass_t(ft_engine *g, bool force, bool dt, bool in_loop, double dt_fi
 
 bool is_surr_mat(int mat) { return mat == 7 || mat == 8; }
 
-// The run loop's element pass with the surrogate: network inputs of every
-// surrogate segment, one inference launch over all their Gauss points, then
-// each segment's element kernel (surrogate stress, or the plain kernel for
-// the other laws).
+// The run loop's element pass with the surrogate: the network's inputs, one
+// inference launch over all Gauss points, the surrogate segments' element
+// kernel, and the plain kernels of the other segments.
 int element_pass_surr(ft_engine *g) {
   const bool audit = g->surr_iter % g->surr_audit_every == 0;
   g->surr_iter += 1;
-  long off = 0;
-  const float *fibf = reinterpret_cast<const float *>(g->fib);
-  {
+  // The surrogate segments follow each other (segments go by material): s0 ..
+  // s1, material 8's elements from e8.
+  size_t s0 = 0;
+  while (s0 < g->segs.size() && !is_surr_mat(g->segs[s0].mat)) ++s0;
+  size_t s1 = s0;
+  while (s1 < g->segs.size() && is_surr_mat(g->segs[s1].mat)) ++s1;
+  int e0 = 0, n = 0;
+  if (s1 > s0) {
+    e0 = g->segs[s0].begin;
+    n = g->segs[s1 - 1].end - e0;
+    const int e8 = g->segs[s1 - 1].mat == 8 ? g->segs[s1 - 1].begin : e0 + n;
     Timed t(g, 2);
-    for (const auto &sg : g->segs) {
-      if (!is_surr_mat(sg.mat)) continue;
-      const int n = sg.end - sg.begin;
-      __bf16 *feat = g->surr_feat + (size_t)off * kSurrFeat;
-      const dim3 grid((n + kBlock - 1) / kBlock);
-      if (sg.mat == 7)
-        hipLaunchKernelGGL(k_surr_features<7>, grid, dim3(kBlock), 0, g->lstream, g->nn, g->ne, g->conn, g->X, g->u,
-                           fibf, sg.begin, sg.end, g->surr_norm, feat, g->ctl, g->parity);
-      else
-        hipLaunchKernelGGL(k_surr_features<8>, grid, dim3(kBlock), 0, g->lstream, g->nn, g->ne, g->conn, g->X, g->u,
-                           fibf, sg.begin, sg.end, g->surr_norm, feat, g->ctl, g->parity);
-      HIPCHK(hipGetLastError());
-      off += 8L * n;
-    }
+    hipLaunchKernelGGL(k_surr_features, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, g->lstream, g->nn, g->ne,
+                       g->conn, g->X, g->u, reinterpret_cast<const float *>(g->fib), e0, e8, e0 + n, g->surr_norm,
+                       g->surr_feat, g->ctl, g->parity);
+    HIPCHK(hipGetLastError());
     int rc = ft::mlp_infer(g->mlp, g->surr_feat, g->surr_gps, g->surr_y, g->lstream);
     if (rc) return rc;
   }
-  off = 0;
-  for (const auto &sg : g->segs) {
+  for (size_t s = 0; s < g->segs.size();) {
+    const auto &sg = g->segs[s];
     int rc;
     if (!is_surr_mat(sg.mat)) {
       if ((rc = force_segment<float, true>(g, sg, sg.waves, true, 0.0, nullptr, 1))) return rc;
+      ++s;
       continue;
     }
-    const int n = sg.end - sg.begin;
-    ElemArgs<float> a = elem_args<float>(g, sg.tile_begin, sg.tile_end, true, 0.0, nullptr, 1);
-    a.surr_y = g->surr_y + (size_t)off * kSurrOut;
+    size_t e = s + 1;  // one launch while the tile sizes agree
+    while (e < s1 && g->segs[e].tile == sg.tile) ++e;
+    const int t0 = sg.tile_begin, t1 = g->segs[e - 1].tile_end;
+    ElemArgs<float> a = elem_args<float>(g, t0, t1, true, 0.0, nullptr, 1);
+    a.surr_y = g->surr_y;
     a.surr_stride = (size_t)n * kSurrOut;
-    a.surr_e0 = sg.begin;
+    a.surr_e0 = e0;
     a.surr_norm = g->surr_norm;
     a.surr_audit = audit ? 1 : 0;
     a.surr_permille = (unsigned)g->surr_permille;
     a.surr_tally = g->surr_tally;
-    a.tile0 = sg.tile_begin;
+    a.tile0 = t0;
     Timed t(g, 0);
-    const dim3 grid(grid_for_tiles(sg.tile_end - sg.tile_begin));
-    if (sg.mat == 7)
-      hipLaunchKernelGGL(k_element_surr<7>, grid, dim3(sg.tile), 0, g->lstream, a);
-    else
-      hipLaunchKernelGGL(k_element_surr<8>, grid, dim3(sg.tile), 0, g->lstream, a);
+    hipLaunchKernelGGL(k_element_surr, dim3(grid_for_tiles(t1 - t0)), dim3(sg.tile), 0, g->lstream, a);
     HIPCHK(hipGetLastError());
-    off += 8L * n;
+    s = e;
   }
   return 0;
 }
