@@ -78,7 +78,7 @@ constexpr int kPlusToMinus = 1 << 26;
 // neighbour along xi lies in another material segment, or across a
 // wavefront boundary of a Prony segment): its xi+ corner j (1, 2, 5, 6 ->
 // j = 0..3) goes to the free xi- slot when bit kExtraFree + j is set, else
-// to its extras entry, which k_pair_extras adds to the owned xi- slot
+// to its extras entry, which k_step_prep adds to the owned xi- slot
 // before the node sum
 constexpr int kExtra = 1 << 25;
 constexpr int kExtraFree = 20;
@@ -129,7 +129,7 @@ struct StepSlot {
   int fresh;       // 1 if the last nodal launch completed a step
   int failed;      // 1 when it stopped because no stable step was left
   // FP32 run loop: best unrefined block minimum of the step (dt_candidate),
-  // 1 once k_motion_states has merged it into dtmin_bits, and the FP32 bits
+  // 1 once k_step_prep has merged it into dtmin_bits, and the FP32 bits
   // of the smallest block minimum beyond the skip margin (far_bits)
   unsigned long long cand_bits;
   int settled;
@@ -1344,7 +1344,7 @@ struct NodalArgs {
   const double *motions;  // per-instance copies, instance i at motion mrange[2 i]
   int n_motions;          // total (stride of mstate)
   const int *mrange;      // per instance: first motion, count (<= kMaxMotions)
-  const MotionT *mstate;  // [3][n_motions], from k_motion_states
+  const MotionT *mstate;  // [3][n_motions], from k_step_prep
   const int4 *tiles;      // node tiles
   int n_tiles;
   Ctl *ctl;               // per instance; ctl[0] also holds the status word
@@ -1458,7 +1458,7 @@ __device__ __forceinline__ void nodal_tile(const NodalArgs<R> &a, const int L) {
   const double t_k = cur.t, t_km1 = cur.t_prev, dt_k = cur.dt;
   double dtmin = bits_to_double(cur.dtmin_bits);
   if (sizeof(R) == 4 && a.cand_geom && !cur.settled) {
-    // FP32 engine, unless k_motion_states has settled the step already: the
+    // FP32 engine, unless k_step_prep has settled the step already: the
     // step's best unrefined element could undercut the refined minimum (it
     // moved up by more than the element kernel's window): its FP64 step from
     // the geometry its tile left (uniform over the block; every block of the
@@ -1479,7 +1479,7 @@ __device__ __forceinline__ void nodal_tile(const NodalArgs<R> &a, const int L) {
   const bool collapse = !(dtmin >= a.failure_dt) || !(dtmin < 1e308);
   const bool go = (t_k < tmax) && (cur.step < cap) && !collapse;
   // this instance's motion states at t_{k-1}, t_k, t_{k+1} (from
-  // k_motion_states, or evaluated here with inline_motions) and, when
+  // k_step_prep, or evaluated here with inline_motions) and, when
   // rotations are present, the parameters motion_apply reads (type,
   // axis, centre), in LDS sized for the run's largest motion count
   // (runs without rotations keep the fixed-size table: its constant strides
@@ -1655,35 +1655,44 @@ __global__ __launch_bounds__(kBlock, ROT ? 6 : 7) void k_nodal(NodalArgs<R> a) {
   nodal_tile<R, W, ROT>(a, xcd_block());
 }
 
-// Scalar state of every motion at t_{k-1}, t_k and t_{k+1} = t_k + dt_{k+1}
-// for the nodal kernel of step k (one small block; the trigonometry of the
-// rotation motions is kept out of the per-node kernel).
-// Motion states of every motion at t_{k-1}, t_k and t_{k+1}.  In the FP32
+// Motion states of every motion at t_{k-1}, t_k and t_{k+1} = t_k + dt_{k+1}
+// for the nodal kernel of step k, by nb blocks (the trigonometry of the
+// rotation motions is kept out of the per-node kernel).  In the FP32
 // engine t_{k+1} needs the step's final minimum: each thread settles a
 // pending candidate itself (the same value), and the first state of each
 // instance's first motion writes it back to the slot and marks the slot
 // settled, so the nodal kernel takes it as final.
-__global__ void k_motion_states(Ctl *ctl, int parity, double factor, const double *motions,
-                                const int *motion_inst, int nm, MotionT *out, const double *cand_geom,
-                                int *status) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 3 * nm; i += gridDim.x * blockDim.x) {
-    const int w = i / nm, k = i % nm;
-    const int inst = motion_inst[k];
-    const StepSlot cur = ctl[inst].slot[parity];
+struct MotionArgs {
+  Ctl *ctl;
+  int parity;
+  double factor;
+  const double *motions;
+  const int *motion_inst;
+  int nm;
+  MotionT *out;
+  const double *cand_geom;
+  int *status;
+};
+
+__device__ inline void motion_states(const MotionArgs &m, int nb) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 3 * m.nm; i += nb * blockDim.x) {
+    const int w = i / m.nm, k = i % m.nm;
+    const int inst = m.motion_inst[k];
+    const StepSlot cur = m.ctl[inst].slot[m.parity];
     double dtmin = bits_to_double(cur.dtmin_bits);
-    if (cand_geom) {
+    if (m.cand_geom) {
       if (candidate_pending(cur, dtmin))
         dtmin = merge_candidate(
-            dtmin, candidate_dt(cand_geom + (size_t)kCandStride * (unsigned)(cur.cand_bits & 0xffffffffu)));
+            dtmin, candidate_dt(m.cand_geom + (size_t)kCandStride * (unsigned)(cur.cand_bits & 0xffffffffu)));
       bool bounded = false;
       dtmin = bound_rule(cur, dtmin, &bounded);
-      if (w == 0 && (k == 0 || motion_inst[k - 1] != inst)) {
-        ctl[inst].slot[parity].dtmin_bits = dt_key(dtmin);
-        ctl[inst].slot[parity].settled = 1;  // read only by the nodal kernel
-        if (bounded) atomicOr(status, FT_STATUS_DT_BOUND);
+      if (w == 0 && (k == 0 || m.motion_inst[k - 1] != inst)) {
+        m.ctl[inst].slot[m.parity].dtmin_bits = dt_key(dtmin);
+        m.ctl[inst].slot[m.parity].settled = 1;  // read only by the nodal kernel
+        if (bounded) atomicOr(m.status, FT_STATUS_DT_BOUND);
       }
     }
-    motion_time(motions + FT_MOTION_STRIDE * k, motion_state_time(cur, factor, w, dtmin), out[i]);
+    motion_time(m.motions + FT_MOTION_STRIDE * k, motion_state_time(cur, m.factor, w, dtmin), m.out[i]);
   }
 }
 
@@ -2641,7 +2650,7 @@ struct ft_engine {
   unsigned char *pzero = nullptr;  // per node: slots to zero around passes outside the run loop
   long n_pairs = 0;
   // extras of the partner-less elements (kExtra): values [4 n][3], per
-  // element its first entry, and the (fe offset, entry) pairs k_pair_extras adds
+  // element its first entry, and the (fe offset, entry) pairs k_step_prep adds
   void *xf = nullptr;
   int *xidx = nullptr;
   int2 *xadd = nullptr;
@@ -3251,7 +3260,7 @@ int element_pass(ft_engine *g, bool force, bool dt, bool in_loop, double dt_fixe
 // Motion states of timed motions: on a mesh of at most kInlineMotionTiles
 // node tiles each tile that holds a constrained node evaluates them itself
 // (no separate launch in the step: 27^3 cube, FP64, 445 steps 15.5 -> 14.9
-// ms); on larger meshes k_motion_states evaluates them once per step (on
+// ms); on larger meshes k_step_prep evaluates them once per step (on
 // the 2.0M-hex ellipsoid, whose every node tile holds surface nodes, the
 // in-tile evaluation cost the node update 10 us).
 constexpr int kInlineMotionTiles = 1024;
@@ -3330,15 +3339,44 @@ int launch_nodal_t(ft_engine *g, int mode, int t0, int t1) {
   return 0;
 }
 
+// What the nodal update needs after the element pass: the motion states (the
+// first nbm blocks) and the corner-pair extras (n of them).  One launch where a
+// step has both: each is bound by latency (40 batched instances: 5.2 + 5.0 us as
+// two launches, 5.9 us as one).
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_step_prep(MotionArgs m, int nbm, int n, const int2 *xadd, const R *xf,
+                                                      R *fe) {
+  if ((int)blockIdx.x < nbm) return motion_states(m, nbm);
+  const int i = (blockIdx.x - nbm) * blockDim.x + threadIdx.x;
+  if (i < n) pair_extras(i, xadd, xf, fe);
+}
+
+int launch_step_prep(ft_engine *g, bool extras) {
+  const bool fp32 = g->precision == FT_FP32;
+  const int n = extras && g->paired ? g->n_xadd : 0;
+  const int nbm = g->timed_motions && !inline_motion_states(g)
+                      ? std::max(1, std::min(64, (3 * g->n_motions + kBlock - 1) / kBlock))
+                      : 0;
+  const dim3 grid(nbm + (n + kBlock - 1) / kBlock);
+  if (grid.x == 0) return 0;
+  const MotionArgs m{g->ctl,         g->parity,    g->factor, g->motions,
+                     g->motion_inst, g->n_motions, g->mstate, fp32 ? (const double *)g->cand_geom : nullptr,
+                     g->status};
+  Timed t(g, 2);
+  if (fp32)
+    hipLaunchKernelGGL(k_step_prep<float>, grid, dim3(kBlock), 0, g->lstream, m, nbm, n, g->xadd,
+                       reinterpret_cast<const float *>(g->xf), reinterpret_cast<float *>(g->fe));
+  else
+    hipLaunchKernelGGL(k_step_prep<double>, grid, dim3(kBlock), 0, g->lstream, m, nbm, n, g->xadd,
+                       reinterpret_cast<const double *>(g->xf), reinterpret_cast<double *>(g->fe));
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
 int launch_nodal(ft_engine *g, int mode) {
-  if (g->timed_motions && !inline_motion_states(g)) {
-    Timed t(g, 2);
-    const int nb = std::max(1, std::min(64, (3 * g->n_motions + kBlock - 1) / kBlock));
-    hipLaunchKernelGGL(k_motion_states, dim3(nb), dim3(kBlock), 0, g->lstream, g->ctl, g->parity, g->factor,
-                       g->motions, g->motion_inst, g->n_motions, g->mstate,
-                       g->precision == FT_FP32 ? (const double *)g->cand_geom : nullptr, g->status);
-    HIPCHK(hipGetLastError());
-  }
+  // (kResume credits the step behind it: no element pass, so no extras)
+  int rp = launch_step_prep(g, mode != kResume);
+  if (rp) return rp;
   const int nt = g->n_ntiles;
   int rc = g->precision == FT_FP32 ? launch_nodal_t<float>(g, mode, 0, nt) : launch_nodal_t<double>(g, mode, 0, nt);
   if (rc) return rc;
@@ -3492,26 +3530,6 @@ struct Unpaired {
     (void)zero_slots(g, 1);
   }
 };
-
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_pair_extras(int n, const int2 *xadd, const R *xf, R *fe) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) pair_extras(i, xadd, xf, fe);
-}
-
-int launch_pair_extras(ft_engine *g) {
-  if (!g->paired || g->n_xadd == 0) return 0;
-  Timed t(g, 2);
-  const dim3 grid((g->n_xadd + kBlock - 1) / kBlock);
-  if (g->precision == FT_FP32)
-    hipLaunchKernelGGL(k_pair_extras<float>, grid, dim3(kBlock), 0, g->lstream, g->n_xadd, g->xadd,
-                       reinterpret_cast<const float *>(g->xf), reinterpret_cast<float *>(g->fe));
-  else
-    hipLaunchKernelGGL(k_pair_extras<double>, grid, dim3(kBlock), 0, g->lstream, g->n_xadd, g->xadd,
-                       reinterpret_cast<const double *>(g->xf), reinterpret_cast<double *>(g->fe));
-  HIPCHK(hipGetLastError());
-  return 0;
-}
 
 // einfo's pair bits from bits[e] (1: kPairLeft, 2: kPairRight, 4: kPlusToMinus,
 // 8: kExtra; bits 4-7: kExtraFree + 0..3).
@@ -4479,7 +4497,6 @@ int ft_run_init(ft_engine *g, double tmax, double dt_factor, double failure_dt) 
   // Initial GetForce + CalculateAccelerations (ex9.cpp:89-92); the Prony
   // update of this pass uses dt_1 like the reference's global dt.
   if ((rc = element_pass(g, true, false, true, 0.0, nullptr, 1))) return rc;
-  if ((rc = launch_pair_extras(g))) return rc;
   if ((rc = upload_caps(g, std::vector<int>(g->n_inst, 0)))) return rc;
   if ((rc = launch_nodal(g, kInitial))) return rc;  // stops: state of step 0
   if ((rc = check_status(g))) return rc;
@@ -4493,7 +4510,6 @@ int loop_body(ft_engine *g) {
   g->sample = (g->loop_iter++ % g->timing_every) == 0;
   int rc;
   if ((rc = element_pass(g, true, true, true, 0.0, nullptr, 1))) return rc;
-  if ((rc = launch_pair_extras(g))) return rc;
   // u still holds this step's displacement here (the nodal kernel below
   // advances it): the injury update of ex5.cpp:240 for t_k
   if (g->inj_on && (rc = injury_launch(g, &g->ctl->slot[g->parity], 0.0, 0.0))) return rc;
