@@ -283,11 +283,12 @@ __device__ inline uint64_t mix64(uint64_t z) {
 // not depend on how samples are spread over blocks.
 // A step is a chain of small products: bound by latency and by the SiLU
 // evaluations, not by the matrix cores, so the rows are split, not only the
-// samples.  A step at a batch of 1,024 / 4,096 / 65,536: 28 / 40 / 295 us;
-// 59 / 82 / 378 us with 32 samples and all rows per wavefront (4 to a block,
-// weights staged in LDS, SiLU' spilled); 540 us at 4,096 as 37 launches of
-// single products and elementwise passes.  At 2 wavefronts per SIMD (44 bytes
-// of spills) instead of 1, 65,536 takes 295 instead of 323 us, 4,096 the same.
+// samples.  A step at a batch of 1,024 / 4,096 / 65,536: 28 / 35 / 295 us (40
+// at 4,096 before k_mlp_grad's empty blocks went); 59 / 82 / 378 us with 32
+// samples and all rows per wavefront (4 to a block, weights staged in LDS,
+// SiLU' spilled); 540 us at 4,096 as 37 launches of single products and
+// elementwise passes.  At 2 wavefronts per SIMD (44 bytes of spills) instead of
+// 1, 65,536 takes 295 instead of 323 us, 4,096 the same.
 constexpr int kTrainTile = 32;      // samples per block
 constexpr int kTrainThreads = 256;  // 4 wavefronts x 32 rows of a layer
 constexpr int kGradChunk = 256;     // samples per weight-gradient block
@@ -476,20 +477,22 @@ __global__ __launch_bounds__(kTrainThreads, 2) void k_mlp_train(TrainArgs g) {
   }
 }
 
-// Weight and bias gradients from k_mlp_train's arrays.  Blocks (x, z): x < 14:
-// weight gradients of samples [256 z, + 256), dW_l[o][i] = sum_s dZ_l[o][s]
-// A_{l-1}[i][s], a 32x32 tile per wavefront (layer 0: x 0, one output tile per
-// wavefront; layers 1-3: x 1-12, an output tile each, an input tile per
-// wavefront; layer 4: x 13), into parts[z].  x >= 14 (z = 0): the bias
-// gradients, one row of dZ each, summed in a fixed order into db.
+// Weight and bias gradients from k_mlp_train's arrays.  The first kDzRows
+// blocks: the bias gradients, one row of dZ each, summed in a fixed order into
+// db.  Then 14 blocks x per 256 samples z: weight gradients of samples [256 z,
+// + 256), dW_l[o][i] = sum_s dZ_l[o][s] A_{l-1}[i][s], a 32x32 tile per
+// wavefront (layer 0: x 0, one output tile per wavefront; layers 1-3: x 1-12,
+// an output tile each, an input tile per wavefront; layer 4: x 13), into
+// parts[z].  (Numbered through: as a grid of (14 + kDzRows) x chunks all but
+// the first chunk's bias blocks were empty; a training step at a batch of 4,096
+// / 16,384: 40 / 68 us, now 35 / 63 us.)
 constexpr int kGradTiles = 14;
 __global__ __launch_bounds__(256) void k_mlp_grad(const __bf16 *at, const __bf16 *dzb, const float *dz, size_t ld,
                                                   float *parts, float *db) {
-  const int x = blockIdx.x, w = threadIdx.x >> 6;
-  if (x >= kGradTiles) {
-    if (blockIdx.y) return;
+  const int w = threadIdx.x >> 6;
+  if (blockIdx.x < kDzRows) {
     __shared__ float sh[256];
-    const float *src = dz + (size_t)(x - kGradTiles) * ld;
+    const float *src = dz + (size_t)blockIdx.x * ld;
     float q = 0.0f;
     for (size_t k = threadIdx.x; k < ld; k += 256) q += src[k];
     sh[threadIdx.x] = q;
@@ -498,15 +501,16 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const __bf16 *at, const __bf16
       if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
       __syncthreads();
     }
-    if (threadIdx.x == 0) db[x - kGradTiles] = sh[0];
+    if (threadIdx.x == 0) db[blockIdx.x] = sh[0];
     return;
   }
+  const int x = (blockIdx.x - kDzRows) % kGradTiles, z = (blockIdx.x - kDzRows) / kGradTiles;
   const int l = x == 0 ? 0 : (x == 13 ? 4 : 1 + (x - 1) / 4);
   const int ot = x == 0 ? w : (x == 13 ? 0 : (x - 1) % 4), it = x == 0 ? 0 : w;
   const int in = layer_in(l), out = layer_out(l);
   const int lane = threadIdx.x & 63, h = lane >> 5, c32 = lane & 31;
   const int r = 32 * ot + c32, c = 32 * it + c32;
-  const size_t s0 = (size_t)blockIdx.y * kGradChunk + 8 * h;
+  const size_t s0 = (size_t)z * kGradChunk + 8 * h;
   const __bf16 *ap = dzb + (size_t)(l * kMlpHid + r) * ld + s0;
   const __bf16 *bp = at + (size_t)((l == 0 ? 0 : kMlpIn + (l - 1) * kMlpHid) + c) * ld + s0;
   const bf16x8 zero8 = {};
@@ -520,7 +524,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const __bf16 *at, const __bf16
 #pragma unroll
   for (int k = 0; k < kGradChunk / 16; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], b[k], acc, 0, 0, 0);
   if (c >= in) return;
-  float *dst = parts + (size_t)blockIdx.y * kParams + w_off(l) + c;
+  float *dst = parts + (size_t)z * kParams + w_off(l) + c;
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     const int o = 32 * ot + 8 * (e >> 2) + 4 * h + (e & 3);
@@ -638,7 +642,7 @@ int train_batch(MlpNet *net, const __bf16 *x, const float *t, long n_data, uint6
   hipLaunchKernelGGL(k_mlp_train, dim3((unsigned)(ld / kTrainTile)), dim3(kTrainThreads), 0, st, g);
   MCHK(hipGetLastError());
   const int nz = (int)(ld / kGradChunk);
-  hipLaunchKernelGGL(k_mlp_grad, dim3(kGradTiles + kDzRows, nz), dim3(256), 0, st, net->at, net->dzb, net->dz, ld,
+  hipLaunchKernelGGL(k_mlp_grad, dim3(kDzRows + kGradTiles * nz), dim3(256), 0, st, net->at, net->dzb, net->dz, ld,
                      net->parts, net->db);
   MCHK(hipGetLastError());
   hipLaunchKernelGGL(k_mlp_update, dim3(blocks(kParams)), dim3(256), 0, st, net->parts, nz, net->db, net->G,
