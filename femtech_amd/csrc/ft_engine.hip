@@ -2765,7 +2765,8 @@ struct ft_engine {
   long surr_gps = 0;
   int surr_audit_every = 100, surr_permille = 10;
   long surr_iter = 0;
-  double *surr_tally = nullptr;
+  double *surr_tally = nullptr;  // 6 per element tile, surr_tally_rows tiles (grow_surr_tally)
+  int surr_tally_rows = 0;
   float *ds_x = nullptr, *ds_t = nullptr;
   long ds_n = 0, ds_cap = 0;
   // timing: every `timing_every`-th step of the run loop is timed (sample)
@@ -3652,6 +3653,30 @@ int build_pairs(ft_engine *g) {
   return 0;
 }
 
+// The surrogate's audit tallies, once they exist, hold a row for each of
+// `rows` element tiles: a change of tile size or force layout after
+// ft_surrogate_enable can make more tiles than it saw.  The rows gathered so
+// far are kept (ft_surrogate_stats only sums them).
+int grow_surr_tally(ft_engine *g, int rows) {
+  if (!g->surr_tally || rows <= g->surr_tally_rows) return 0;
+  double *t = nullptr;
+  int rc = dalloc(&t, 6 * (size_t)rows);
+  if (rc) return rc;
+  const size_t old = 6 * (size_t)g->surr_tally_rows;
+  hipError_t e = hipMemsetAsync(t + old, 0, (6 * (size_t)rows - old) * sizeof(double), g->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(t, g->surr_tally, old * sizeof(double), hipMemcpyDeviceToDevice, g->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
+  if (e != hipSuccess) {
+    (void)hipFree(t);
+    return fail(FT_ERR_HIP, "audit tallies: %s", hipGetErrorString(e));
+  }
+  (void)hipFree(g->surr_tally);
+  g->surr_tally = t;
+  g->surr_tally_rows = rows;
+  return 0;
+}
+
 // Element tiles: at most sg.tile consecutive elements of one material
 // segment (internal order) and one instance.
 int build_element_tiles(ft_engine *g) {
@@ -3670,8 +3695,9 @@ int build_element_tiles(ft_engine *g) {
       }
   }
   std::vector<int4> et;
-  for (auto &sg : g->segs) {
-    sg.tile_begin = (int)et.size();
+  std::vector<int> tile0;  // first tile of each segment
+  for (const auto &sg : g->segs) {
+    tile0.push_back((int)et.size());
     const bool seg_shadows = shadows && sg.mat != 5 && sg.mat != 7;
     const int cap = seg_shadows ? sg.tile / 64 * 63 : sg.tile;
     for (int i = sg.begin; i < sg.end;) {
@@ -3683,7 +3709,13 @@ int build_element_tiles(ft_engine *g) {
                                              (sg.mat << kTileMat)));
       i = j;
     }
-    sg.tile_end = (int)et.size();
+  }
+  int rc = grow_surr_tally(g, (int)et.size());  // (before the launches' tile ranges change)
+  if (rc) return rc;
+  tile0.push_back((int)et.size());
+  for (size_t s = 0; s < g->segs.size(); ++s) {
+    g->segs[s].tile_begin = tile0[s];
+    g->segs[s].tile_end = tile0[s + 1];
   }
   for (void *p : {(void *)g->etiles, (void *)g->cand_geom})
     if (p) (void)hipFree(p);
@@ -3691,7 +3723,6 @@ int build_element_tiles(ft_engine *g) {
   g->cand_geom = nullptr;
   g->n_etiles = (int)et.size();
   g->h_etiles = et;
-  int rc;
   if ((rc = dalloc(&g->etiles, et.size())) || (rc = dalloc(&g->cand_geom, kCandStride * et.size())))
     return rc;
   HIPCHK(hipMemcpy(g->etiles, et.data(), et.size() * sizeof(int4), hipMemcpyHostToDevice));
@@ -5107,10 +5138,13 @@ int ft_surrogate_enable(ft_engine *g, int enable, int audit_every, int audit_per
       return rc;
     g->surr_gps = gps;
   }
+  g->surr_on = false;  // until the tallies below exist
   if (g->surr_tally) (void)hipFree(g->surr_tally);
   g->surr_tally = nullptr;
+  g->surr_tally_rows = 0;
   int rc;
   if ((rc = dalloc(&g->surr_tally, (size_t)std::max(1, g->n_etiles) * 6))) return rc;
+  g->surr_tally_rows = std::max(1, g->n_etiles);
   HIPCHK(hipMemset(g->surr_tally, 0, (size_t)std::max(1, g->n_etiles) * 6 * sizeof(double)));
   g->surr_audit_every = audit_every;
   g->surr_permille = audit_permille;
@@ -5123,7 +5157,7 @@ int ft_surrogate_stats(ft_engine *g, double out[6]) {
   if (!g || !out) return fail(FT_ERR_ARG, "null argument");
   for (int k = 0; k < 6; ++k) out[k] = 0.0;
   if (!g->surr_tally) return 0;
-  std::vector<double> t((size_t)std::max(1, g->n_etiles) * 6);
+  std::vector<double> t((size_t)g->surr_tally_rows * 6);
   HIPCHK(hipStreamSynchronize(g->stream));
   HIPCHK(hipMemcpy(t.data(), g->surr_tally, t.size() * sizeof(double), hipMemcpyDeviceToHost));
   double v[6] = {0, 0, 0, 0, 0, 0};
@@ -5291,9 +5325,13 @@ int ft_set_segment_shape(ft_engine *g, int segment, int waves, int tile) {
     return fail(FT_ERR_ARG, "occupancy variant %d not available", waves);
   if (tile != 64 && tile != 128 && tile != 256) return fail(FT_ERR_ARG, "tile size must be 64, 128 or 256");
   drop_graphs(g);
-  g->segs[segment].waves = waves;
-  g->segs[segment].tile = tile;
-  return build_element_tiles(g);
+  auto &sg = g->segs[segment];
+  const int waves0 = sg.waves, tile0 = sg.tile;
+  sg.waves = waves;
+  sg.tile = tile;
+  const int rc = build_element_tiles(g);
+  if (rc) sg.waves = waves0, sg.tile = tile0;
+  return rc;
 }
 
 int ft_set_timing(ft_engine *g, int enable) {
