@@ -337,14 +337,21 @@ __device__ __forceinline__ void tile_to_operands(const float (&v)[16], bf16x8 (&
 }
 
 // SiLU and its derivative as z / (1 + e^-z) and s (1 + z (1 - s)), s = 1 / (1 +
-// e^-z): the reciprocal refined to full precision serves both divisions.
+// e^-z): the reciprocal refined to full precision serves both divisions.  It is
+// taken of the denominator scaled down by a power of two: from 2^126 on (z below
+// -87) a reciprocal is too small for the instruction, but not the quotients.
+// (The same with the scaling only where it is needed and div_fixup for infinite
+// operands: 428 bytes of spills instead of 44, 376 against 300 us per step at a
+// batch of 65,536.)
 __device__ __forceinline__ void silu_both(float z, float &v, float &d) {
-  const float ez = 1.0f + __expf(-z);
-  float s = __builtin_amdgcn_rcpf(ez);
-  const float r = fmaf(fmaf(-ez, s, 1.0f), s, s);
-  s = ez < 1e30f ? r : 0.0f;  // (beyond, both vanish in FP32)
-  const float q = z * s;
-  v = ez < 1e30f ? fmaf(fmaf(-q, ez, z), s, q) : z * 0.0f;
+  constexpr float kDown = 0x1p-64f;
+  const float t = __expf(-z), ez = 1.0f + t, e = fmaf(t, kDown, kDown);
+  float s = __builtin_amdgcn_rcpf(e);
+  s = fmaf(fmaf(-e, s, 1.0f), s, s) * kDown;
+  const bool finite = ez < INFINITY;
+  s = finite ? s : 0.0f;
+  const float q = z * s, w = fmaf(fmaf(-q, ez, z), s, q);
+  v = z > 0x1p24f ? z : (finite ? w : q);  // (z itself, also where it is infinite)
   d = s * (1.0f + z * (1.0f - s));
 }
 
