@@ -4762,6 +4762,7 @@ int ft_snapshot_end(ft_engine *g, double *u, double *time, int *step) {
 
 int ft_get_state(ft_engine *g, double *u, double *v, double *a, double *fi) {
   if (!g) return fail(FT_ERR_ARG, "null engine");
+  if (!u && !v && !a && !fi) HIPCHK(hipStreamSynchronize(g->stream));  // (each read-back below waits itself)
   int rc0;
   if (u && (rc0 = d2h_nodal(g, u, g->u))) return rc0;
   if (v && (rc0 = d2h_nodal(g, v, g->vs))) return rc0;
