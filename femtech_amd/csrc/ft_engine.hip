@@ -43,6 +43,8 @@ int fail(int code, const char *fmt, ...) {
   vsnprintf(buf, sizeof(buf), fmt, ap);
   va_end(ap);
   g_err = buf;
+  // reported here, so not by the check behind a later launch
+  if (code == FT_ERR_HIP || code == FT_ERR_ALLOC) (void)hipGetLastError();
   return code;
 }
 

@@ -42,6 +42,8 @@ int mfail(int code, const char *fmt, ...) {
   vsnprintf(buf, sizeof(buf), fmt, ap);
   va_end(ap);
   ft_internal_set_error(buf);
+  // reported here, so not by the check behind a later launch
+  if (code == FT_ERR_HIP || code == FT_ERR_ALLOC) (void)hipGetLastError();
   return code;
 }
 
