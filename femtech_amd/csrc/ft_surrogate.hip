@@ -778,9 +778,10 @@ int mlp_train(MlpNet *net, const __bf16 *x, const float *t, long n_data, int ste
   for (int k = 0; k < steps; ++k) {
     const uint64_t key = seed * 0x9E3779B97F4A7C15ull ^ ((uint64_t)k << 20);
     const float lr_k = lr * (0.02f + 0.98f * 0.5f * (1.0f + cosf(3.14159265f * (float)k / (float)steps)));
-    net->adam_t += 1;
-    const AdamStep a{lr_k, (float)(1.0 / (1.0 - pow(0.9, net->adam_t))), (float)(1.0 / (1.0 - pow(0.999, net->adam_t)))};
+    const int at = net->adam_t + 1;
+    const AdamStep a{lr_k, (float)(1.0 / (1.0 - pow(0.9, at))), (float)(1.0 / (1.0 - pow(0.999, at)))};
     if ((rc = train_batch(net, x, t, n_data, key, batch, &a, st))) return rc;
+    net->adam_t = at;  // (a step that could not be launched is none)
     // the loss is read back (a synchronisation) only over the last 1 % of steps
     if (final_loss && k >= steps - std::max(1, steps / 100)) {
       double l = 0.0;
