@@ -3138,15 +3138,27 @@ int launch_waves(ft_engine *g, size_t s0, size_t s1, bool force, bool dt, bool i
 }
 
 // End of the run of FP32 segments from s on that k_element_merged takes in the
-// run loop (s: none): neighbours of default launch shape, the longest run
-// within 50,000 + 70,000 elements per segment.  Alone, each launch of a small
-// segment costs its law's latency (16 to 33 us); together they share it, but
-// run at two wavefronts per SIMD.  Measured, us of element launches per step,
-// each / merged, for equal parts of one mesh: neo-Hookean and linear elastic
-// 31.0 / 16.5 at 32,768 elements in all, 32.9 / 20.5 at 97,336, 45.1 / 52.7
-// at 262,144; linear elastic, Ogden + Prony and anisotropic HGO 61.1 / 30.8,
-// 64.1 / 37.8, 77.6 / 82.9; five laws 82.8 / 22.7, 85.5 / 28.8, 90.8 / 65.7,
-// and 109.5 / 123.7 at 512,000.
+// run loop (s: none): neighbours of default launch shape, the longest run of n
+// segments within merge_limit(n) elements.  Alone, each launch of a small
+// segment costs its law's latency (12 to 33 us); together they share it, but
+// run at two wavefronts per SIMD: the launch's time steps up with every 129,000
+// elements, one round of resident blocks, where the separate launches of laws
+// held to 4 wavefronts grow by half of that.  The more segments, the more
+// latency pays for such a round.  Measured, us of element launches per step,
+// each / merged.  Two segments, one of 2,000 elements, 140,608 / 181,944 in all:
+// neo-Hookean 35.9 / 32.5 and 37.0 / 41.3, St Venant-Kirchhoff 36.1 / 32.7 and
+// 36.6 / 42.5, HGO + Prony 53.7 / 50.9 and 58.9 / 63.8, Ogden + Prony 65.0 / 55.3
+// and 69.2 / 64.4.  Three (rigid, neo-Hookean, HGO + Prony, the last two alike),
+// 230,000 / 258,000: 64.7 / 62.0, 64.3 / 63.3; (rigid, neo-Hookean, St Venant-
+// Kirchhoff) 51.7 / 44.7, 52.1 / 49.9.  Four (rigid, neo-Hookean, St Venant-
+// Kirchhoff, HGO + Prony in equal parts), 258,000 / 328,000: 71.2 / 59.3, 79.5 /
+// 84.2.  Five (with linear elastic), 385,000 / 400,000: 98.4 / 90.3, 99.8 / 103.9.
+// Six (with Ogden), 470,000: 126.0 / 113.4; all nine, 680,000: 196.9 / 159.5.
+long merge_limit(long n) {
+  constexpr long kFew[] = {0, 0, 150000, 250000, 280000, 385000};
+  return n <= 5 ? kFew[n] : 50000 + 70000 * n;
+}
+
 size_t merge_run(const ft_engine *g, size_t s) {
   size_t best = s;
   long total = 0;
@@ -3155,7 +3167,7 @@ size_t merge_run(const ft_engine *g, size_t s) {
     if (sg.waves != 0 || sg.tile != kBlock) break;
     const long n = (long)(s1 - s) + 1;
     total += sg.end - sg.begin;
-    if (n > 1 && total <= 50000 + 70000 * n) best = s1 + 1;
+    if (n > 1 && total <= merge_limit(n)) best = s1 + 1;
   }
   return best;
 }
