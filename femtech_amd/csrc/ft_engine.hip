@@ -3077,7 +3077,8 @@ int force_segment(ft_engine *g, const ft_engine::Seg &sg, int waves, bool in_loo
 // k_element / k_element_waves at 1,000, 8,000, 32,768 and 97,336 elements:
 // neo-Hookean 16.8 / 11.0, 17.3 / 11.6, 18.7 / 21.3, 28.8 / 39.8; HGO + Prony
 // 27.8 / 13.4, 28.9 / 15.5, 31.4 / 29.4, 58.6 / 70.9; Ogden + Prony 83.3 /
-// 31.4, 95.0 / 29.1, 60.8 / 37.9, 90.0 / 88.5; anisotropic HGO 23.5 / 11.9,
+// 31.4, 95.0 / 29.1, 55.9 / 37.2, 86.6 / 83.2, and 88.4 / 93.5 at 103,823, 88.3 /
+// 104.5 at 115,248; Ogden 81.0 / 81.1 at 89,100; anisotropic HGO 23.5 / 11.9,
 // 23.7 / 12.1, 25.4 / 23.3, 42.0 / 44.3.  The launch shapes of
 // ft_set_segment_shape and ft_autotune apply to k_element only.
 struct WaveCost {
@@ -3090,7 +3091,7 @@ WaveCost wave_cost(int mat) {
     case 4: return {19, 65000};
     case 5: return {26, 60000};
     case 6: return {40, 120000};
-    case 7: return {60, 150000};
+    case 7: return {60, 118000};
     case 8: return {21, 100000};
     default: return {15, 80000};
   }
