@@ -425,7 +425,7 @@ struct ElemArgs {
 // leave one wave); the FP32 Prony laws (5, 7), Ogden's law (6), the fibre law
 // (8) and the FP64 Prony laws are not held.  WAVES > 0 overrides it (the FP32 run-loop
 // instances are compiled for WAVES = 1..5 and the tuner picks one per
-// material segment).
+// material segment; FP64: one_wave).
 #ifndef FT_ELEM_WAVES_FP32
 #define FT_ELEM_WAVES_FP32 4
 #endif
@@ -2998,6 +2998,14 @@ int launch_element(ft_engine *g, int t0, int t1, bool in_loop, double dt_fixed, 
 // A material segment's force kernel with the segment's launch shape: its
 // tile size is the block size; its occupancy variant applies to the FP32
 // force + dt kernel (the run loop's), the others use the default.
+//
+// FP64, isotropic and anisotropic HGO: held to 2 wavefronts per SIMD they spill
+// registers, which pays only where a SIMD gets a second wavefront.  us per
+// launch held / not held: isotropic 25.8 / 24.2 at 64,000 elements, 35.5 / 38.1
+// at 67,200, 106 / 121 at 405,000; anisotropic 29.1 / 25.4, 40.7 / 40.4, 130 / 132.
+constexpr long kSimds = 1024;
+inline bool one_wave(int tiles, int tile) { return (long)tiles * (tile / 64) <= kSimds; }
+
 template <typename R, bool DT, int MAT>
 int force_segment_mat(ft_engine *g, const ft_engine::Seg &sg, int waves, bool in_loop, double dt_fixed,
                       unsigned long long *dtbits, int update_hist) {
@@ -3011,6 +3019,10 @@ int force_segment_mat(ft_engine *g, const ft_engine::Seg &sg, int waves, bool in
       case 5: return launch_element<R, true, DT, MAT, 5>(g, t0, t1, in_loop, dt_fixed, dtbits, update_hist, b);
       default: break;
     }
+  }
+  if constexpr (sizeof(R) == 8 && (MAT == 4 || MAT == 8)) {
+    if (one_wave(t1 - t0, b))
+      return launch_element<R, true, DT, MAT, 1>(g, t0, t1, in_loop, dt_fixed, dtbits, update_hist, b);
   }
   return launch_element<R, true, DT, MAT>(g, t0, t1, in_loop, dt_fixed, dtbits, update_hist, b);
 }
@@ -3079,7 +3091,7 @@ int force_segment(ft_engine *g, const ft_engine::Seg &sg, int waves, bool in_loo
 // 27.8 / 13.4, 28.9 / 15.5, 31.4 / 29.4, 58.6 / 70.9; Ogden + Prony 83.3 /
 // 31.4, 95.0 / 29.1, 55.9 / 37.2, 86.6 / 83.2, and 88.4 / 93.5 at 103,823, 88.3 /
 // 104.5 at 115,248; Ogden 81.0 / 81.1 at 89,100; anisotropic HGO 23.5 / 11.9,
-// 23.7 / 12.1, 25.4 / 23.3, 42.0 / 44.3.  The launch shapes of
+// 23.7 / 12.1, 22.4 / 22.7, 42.0 / 44.3.  The launch shapes of
 // ft_set_segment_shape and ft_autotune apply to k_element only.
 struct WaveCost {
   double alone;  // us
@@ -3092,7 +3104,7 @@ WaveCost wave_cost(int mat) {
     case 5: return {26, 60000};
     case 6: return {40, 120000};
     case 7: return {60, 118000};
-    case 8: return {21, 100000};
+    case 8: return {21, 65000};
     default: return {15, 80000};
   }
 }
