@@ -506,9 +506,9 @@ class Engine:
         _check(self._lib.ft_set_segment_shape(self._h, int(segment), int(waves), int(tile)))
 
     def autotune(self, repeats=5):
-        """Times every element-kernel launch shape per material segment and
-        keeps the fastest.  Returns rows (material, elements, waves, tile,
-        best us, default-shape us)."""
+        """Times every element-kernel launch shape per material segment, and
+        the launches that small segments share, and keeps the fastest.  Returns
+        rows (material, elements, waves, tile, best us, default-shape us)."""
         n = len(self.segments())
         rep = np.zeros(6 * n)
         cnt = ctypes.c_int(0)

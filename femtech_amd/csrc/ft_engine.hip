@@ -3185,8 +3185,10 @@ size_t merge_run(const ft_engine *g, size_t s) {
   return best;
 }
 
-int launch_merged(ft_engine *g, size_t s0, size_t s1) {
-  const ElemArgs<float> a = elem_args<float>(g, g->segs[s0].tile_begin, g->segs[s1 - 1].tile_end, true, 0.0, nullptr, 1);
+int launch_merged(ft_engine *g, size_t s0, size_t s1, bool in_loop = true, double dt_fixed = 0.0,
+                  unsigned long long *dtbits = nullptr) {
+  const ElemArgs<float> a =
+      elem_args<float>(g, g->segs[s0].tile_begin, g->segs[s1 - 1].tile_end, in_loop, dt_fixed, dtbits, 1);
   if (a.n_tiles <= 0) return 0;
   Timed t(g, 0);
   hipLaunchKernelGGL(k_element_merged, dim3(grid_for_tiles(a.n_tiles)), dim3(kBlock), 0, g->lstream, a);
@@ -5223,6 +5225,12 @@ int ft_set_graph(ft_engine *g, int steps) {
 // scratch minimum and a scratch copy of the Prony history (updated as in the
 // loop, so its traffic is part of the timing); the status word is restored,
 // so tuning between run calls leaves the run unchanged.
+//
+// Segments that share a launch at the default shape (wave_run, merge_run) are
+// timed in that launch: FP64 ones stay in it, whatever their shape, so theirs
+// is the default; FP32 ones stay in it unless the launches of their own, each
+// at its best shape, are faster together (five laws on 33k elements: 22.7 us
+// against 80 us or more).
 int ft_autotune(ft_engine *g, int repeats, double *report, int *n_segments) {
   if (!g) return fail(FT_ERR_ARG, "null engine");
   if (repeats < 1) return fail(FT_ERR_ARG, "repeats < 1");
@@ -5251,12 +5259,7 @@ int ft_autotune(ft_engine *g, int repeats, double *report, int *n_segments) {
   }
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) rc = fail(FT_ERR_HIP, "event creation failed");
-  auto time_one = [&](size_t si, int waves, double &us) -> int {
-    const ft_engine::Seg sg = g->segs[si];
-    auto launch = [&]() {
-      return fp32 ? force_segment<float, true>(g, sg, waves, false, 1e-7, g->dtbits, 1)
-                  : force_segment<double, true>(g, sg, waves, false, 1e-7, g->dtbits, 1);
-    };
+  auto time_launch = [&](auto launch, double &us) -> int {
     int r;
     if ((r = launch())) return r;  // warm-up
     HIPCHK(hipEventRecord(e0, g->stream));
@@ -5269,11 +5272,49 @@ int ft_autotune(ft_engine *g, int repeats, double *report, int *n_segments) {
     us = 1e3 * ms / repeats;
     return 0;
   };
+  auto time_one = [&](size_t si, int waves, double &us) -> int {
+    const ft_engine::Seg sg = g->segs[si];
+    return time_launch(
+        [&]() {
+          return fp32 ? force_segment<float, true>(g, sg, waves, false, 1e-7, g->dtbits, 1)
+                      : force_segment<double, true>(g, sg, waves, false, 1e-7, g->dtbits, 1);
+        },
+        us);
+  };
   const int tiles[3] = {64, 128, 256};
   const size_t ns = g->segs.size();
   std::vector<double> rows(6 * ns, 0.0);
+  // runs of segments [s, shared[s]) that share a launch at the default shape
+  for (auto &sg : g->segs) sg.waves = 0, sg.tile = kBlock;
+  std::vector<size_t> shared(ns, 0);
+  for (size_t s = 0; s < ns; ++s) {
+    const size_t s1 = g->surr_on ? s : fp32 ? merge_run(g, s) : wave_run(g, s);
+    for (size_t k = s; k < s1; ++k) shared[k] = s1;
+    if (s1 > s) s = s1 - 1;
+  }
+  auto time_shared = [&](size_t s0, double &us) -> int {
+    return time_launch(
+        [&]() {
+          return fp32 ? launch_merged(g, s0, shared[s0], false, 1e-7, g->dtbits)
+                      : launch_waves(g, s0, shared[s0], true, true, false, 1e-7, g->dtbits, 1);
+        },
+        us);
+  };
+  auto report_shared = [&](size_t s0, double us) {
+    for (size_t k = s0; k < shared[s0]; ++k) {
+      const double r[6] = {(double)g->segs[k].mat, (double)(g->segs[k].end - g->segs[k].begin), 0, kBlock, us, us};
+      std::copy(r, r + 6, &rows[6 * k]);
+    }
+  };
   for (size_t si = 0; si < ns && !rc; ++si) {
     auto &sg = g->segs[si];
+    if (!fp32 && shared[si]) {
+      double us = 0;
+      if ((rc = build_element_tiles(g)) || (rc = time_shared(si, us))) break;
+      report_shared(si, us);
+      si = shared[si] - 1;
+      continue;
+    }
     double best = 1e300, t_def = 0;
     int bw = 0, bt = kBlock;
     for (int tile : tiles) {
@@ -5313,6 +5354,28 @@ int ft_autotune(ft_engine *g, int repeats, double *report, int *n_segments) {
     r[3] = bt;
     r[4] = best;
     r[5] = t_def;
+  }
+  // each FP32 run of small segments: one launch, or theirs
+  for (size_t s0 = 0; s0 < ns && !rc; ++s0) {
+    if (!fp32 || !shared[s0]) continue;
+    const size_t s1 = shared[s0];
+    double apart = 0, us = 0;
+    std::vector<ft_engine::Seg> own(g->segs.begin() + s0, g->segs.begin() + s1);
+    for (size_t k = s0; k < s1; ++k) {
+      apart += rows[6 * k + 4];
+      g->segs[k].waves = 0;
+      g->segs[k].tile = kBlock;
+    }
+    if ((rc = build_element_tiles(g)) || (rc = time_shared(s0, us))) break;
+    if (us <= apart) {
+      report_shared(s0, us);
+    } else {
+      for (size_t k = s0; k < s1; ++k) {
+        g->segs[k].waves = own[k - s0].waves;
+        g->segs[k].tile = own[k - s0].tile;
+      }
+    }
+    s0 = s1 - 1;
   }
   if (!rc) rc = build_element_tiles(g);
   if (hist_copy) {

@@ -350,9 +350,11 @@ int ft_injury_results(ft_engine *eng, double out[21], int *flags);
  * default shape (256 elements per block, compiler-chosen occupancy), and
  * keeps the fastest; occupancy variants that spill more than 128 bytes of
  * registers per lane to scratch memory are skipped.  Small segments at the
- * default shape share a launch in the run loop; one with another shape keeps
- * its own.  report (may be NULL): 6 doubles per segment = material,
- * elements, waves, tile, best us per launch, default-shape us per launch.
+ * default shape share a launch in the run loop; in FP32 one with another shape
+ * keeps its own.  They keep the default shape unless launches of their own (FP32)
+ * are faster together.  report (may be NULL): 6 doubles per segment = material,
+ * elements, waves, tile, best us per launch, default-shape us per launch (of
+ * segments left to share a launch: that launch's time in both).
  * The run state is unchanged (the Prony history is not advanced).
  * ft_get_segments: desc (may be NULL) gets 5 ints per segment = material,
  * first and end element (internal, grouped order), waves (0 = default), tile.
