@@ -30,6 +30,12 @@ struct PartDev {
   double kappa;  // fibre dispersion (material 8)
 };
 
+// Sums of products.  FP64: with the fused operations written out, so that a
+// kernel's results do not hang on which of two products the compiler fuses into
+// their sum (it differed between the kernels that share these routines: a mesh
+// in a batch, which takes k_element, and alone, which takes k_element_waves,
+// came out a last bit apart).  mul_: a product that is not fused into a later
+// sum.  FP32: the plain expressions, the choice left to the compiler.
 template <typename R> struct Num;
 template <> struct Num<float> {
   // log(1 + x): 7-term series for |x| < 1/16 (truncation < 4e-11 relative),
@@ -48,6 +54,13 @@ template <> struct Num<float> {
     return log1pf(x);
   }
   __host__ __device__ static float fma_(float a, float b, float c) { return fmaf(a, b, c); }
+  __host__ __device__ static float mul_(float a, float b) { return a * b; }
+  __host__ __device__ static float add_prod(float c, float a, float b) { return c + a * b; }
+  __host__ __device__ static float prod_add(float a, float b, float c) { return a * b + c; }
+  __host__ __device__ static float dot2(float a, float b, float c, float d) { return a * b + c * d; }
+  __host__ __device__ static float dot3(float a, float b, float c, float d, float e, float f) {
+    return a * b + c * d + e * f;
+  }
   // exp(x) - 1: 8-term series for |x| < 1/16 (truncation < 1e-13
   // relative), the library routine otherwise
   __host__ __device__ static float expm1_(float x) {
@@ -94,6 +107,18 @@ template <> struct Num<float> {
 template <> struct Num<double> {
   __host__ __device__ static double log1p_(double x) { return log1p(x); }
   __host__ __device__ static double fma_(double a, double b, double c) { return fma(a, b, c); }
+  __host__ __device__ static double mul_(double a, double b) {
+#ifdef __clang__
+#pragma clang fp contract(off)
+#endif
+    return a * b;
+  }
+  __host__ __device__ static double add_prod(double c, double a, double b) { return fma(a, b, c); }
+  __host__ __device__ static double prod_add(double a, double b, double c) { return fma(a, b, c); }
+  __host__ __device__ static double dot2(double a, double b, double c, double d) { return fma(c, d, a * b); }
+  __host__ __device__ static double dot3(double a, double b, double c, double d, double e, double f) {
+    return fma(e, f, fma(c, d, a * b));
+  }
   __host__ __device__ static double expm1_(double x) { return expm1(x); }
   __host__ __device__ static double exp_(double x) { return exp(x); }
   __host__ __device__ static double sqrt_(double x) { return sqrt(x); }
@@ -193,8 +218,8 @@ __host__ __device__ inline Sym<R> green_lagrange(const R H[3][3]) {
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
     int i = I[k], j = J[k];
-    R hth = H[0][i] * H[0][j] + H[1][i] * H[1][j] + H[2][i] * H[2][j];
-    E.v[k] = R(0.5) * (H[i][j] + H[j][i] + hth);
+    R hth = Num<R>::dot3(H[0][i], H[0][j], H[1][i], H[1][j], H[2][i], H[2][j]);
+    E.v[k] = Num<R>::mul_(R(0.5), H[i][j] + H[j][i] + hth);
   }
   return E;
 }
@@ -223,9 +248,9 @@ __host__ __device__ inline Sym<R> sym_mul(const Sym<R> &A, const Sym<R> &T, R s)
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
     int i = I[k], j = J[k];
-    R acc = sym_at(A, i, 0) * sym_at(T, 0, j) + sym_at(A, i, 1) * sym_at(T, 1, j) +
-            sym_at(A, i, 2) * sym_at(T, 2, j);
-    S.v[k] = acc * s;
+    R acc = Num<R>::dot3(sym_at(A, i, 0), sym_at(T, 0, j), sym_at(A, i, 1), sym_at(T, 1, j), sym_at(A, i, 2),
+                         sym_at(T, 2, j));
+    S.v[k] = Num<R>::mul_(acc, s);
   }
   return S;
 }
@@ -291,12 +316,12 @@ __host__ __device__ inline void sym_eig3(const Sym<R> &m, R w[3], R V[3][3]) {
       a[p][q] = a[q][p] = R(0);
       const R aop = a[o][p], aoq = a[o][q];
       a[o][p] = a[p][o] = c * aop - sn * aoq;
-      a[o][q] = a[q][o] = sn * aop + c * aoq;
+      a[o][q] = a[q][o] = Num<R>::dot2(sn, aop, c, aoq);
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         const R vp = V[k][p], vq = V[k][q];
         V[k][p] = c * vp - sn * vq;
-        V[k][q] = sn * vp + c * vq;
+        V[k][q] = Num<R>::dot2(sn, vp, c, vq);
       }
     }
     if constexpr (sizeof(R) == 4) {
@@ -319,7 +344,7 @@ __host__ __device__ inline Sym<R> b_minus_identity(const R H[3][3]) {
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
     const int i = I[k], j = J[k];
-    bm.v[k] = H[i][j] + H[j][i] + (H[i][0] * H[j][0] + H[i][1] * H[j][1] + H[i][2] * H[j][2]);
+    bm.v[k] = H[i][j] + H[j][i] + Num<R>::dot3(H[i][0], H[j][0], H[i][1], H[j][1], H[i][2], H[j][2]);
   }
   return bm;
 }
@@ -351,7 +376,7 @@ __host__ __device__ inline void ogden_tau(const PartDev &pp, const Sym<R> &bm, R
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
     const int i = I[k], j = J[k];
-    tau.v[k] = t[0] * V[i][0] * V[j][0] + t[1] * V[i][1] * V[j][1] + t[2] * V[i][2] * V[j][2];
+    tau.v[k] = Num<R>::dot3(t[0] * V[i][0], V[j][0], t[1] * V[i][1], V[j][1], t[2] * V[i][2], V[j][2]);
   }
   p = R(0.5) * K * Jm1 * (Jm1 + R(2));
 }
@@ -389,7 +414,7 @@ __host__ __device__ inline bool ogden_iso_series(const PartDev &pp, const R H[3]
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
     const int i = I[k], j = J[k];
-    Z.v[k] = H[i][j] + H[j][i] + (H[0][i] * H[0][j] + H[1][i] * H[1][j] + H[2][i] * H[2][j]);
+    Z.v[k] = H[i][j] + H[j][i] + Num<R>::dot3(H[0][i], H[0][j], H[1][i], H[1][j], H[2][i], H[2][j]);
   }
   {  // C^-1 = adj(C) / J^2
     const R c0 = R(1) + Z.v[0], c1 = R(1) + Z.v[1], c2 = R(1) + Z.v[2];
@@ -411,7 +436,8 @@ __host__ __device__ inline bool ogden_iso_series(const PartDev &pp, const R H[3]
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
     const int i = I[k], j = J[k];
-    Q.v[k] = sym_at(Z, i, 0) * sym_at(Z, j, 0) + sym_at(Z, i, 1) * sym_at(Z, j, 1) + sym_at(Z, i, 2) * sym_at(Z, j, 2);
+    Q.v[k] = Num<R>::dot3(sym_at(Z, i, 0), sym_at(Z, j, 0), sym_at(Z, i, 1), sym_at(Z, j, 1), sym_at(Z, i, 2),
+                          sym_at(Z, j, 2));
   }
   const R i1 = Z.v[0] + Z.v[1] + Z.v[2];
   const R i2 = (Z.v[0] * Z.v[1] - Z.v[5] * Z.v[5]) + (Z.v[0] * Z.v[2] - Z.v[4] * Z.v[4]) + (Z.v[1] * Z.v[2] - Z.v[3] * Z.v[3]);
@@ -440,7 +466,7 @@ __host__ __device__ inline bool ogden_iso_series(const PartDev &pp, const R H[3]
   if (!done) return false;
   Sym<R> M;
 #pragma unroll
-  for (int k = 0; k < 6; ++k) M.v[k] = sb * Z.v[k] + sc * Q.v[k];
+  for (int k = 0; k < 6; ++k) M.v[k] = Num<R>::dot2(sb, Z.v[k], sc, Q.v[k]);
   const R tr = Num<R>::div_c(M.v[0] + M.v[1] + M.v[2], 3.0);
   M.v[0] -= tr;
   M.v[1] -= tr;
@@ -514,8 +540,6 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
     // LinearElastic.cpp:14-70: P = lambda tr(eps) I + 2 mu eps, S = F^-1 P,
     // unsymmetrised, upper triangle kept.
     R trE = H[0][0] + H[1][1] + H[2][2];
-    // (the fused products are written out: left to the compiler, their choice
-    // differed between the kernels that share this routine)
     R P[3][3];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -535,7 +559,7 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
       int i = I[k], j = J[k];
-      S.v[k] = Num<R>::fma_(A[i][2], P[2][j], Num<R>::fma_(A[i][1], P[1][j], A[i][0] * P[0][j])) * iJ;
+      S.v[k] = Num<R>::mul_(Num<R>::fma_(A[i][2], P[2][j], Num<R>::fma_(A[i][1], P[1][j], A[i][0] * P[0][j])), iJ);
     }
     return true;
   }
@@ -547,14 +571,14 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
     const R p = R(0.5) * (lambda + Num<R>::div_c(R(2) * mu, 3.0)) * Jm1 * (Jm1 + R(2));
     ogden_iso(pp, H, Jm1, Sdev, Ci);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) S.v[k] = Sdev.v[k] + p * Ci.v[k];
+    for (int k = 0; k < 6; ++k) S.v[k] = Num<R>::add_prod(Sdev.v[k], p, Ci.v[k]);
     if (mat == 7 && use_hist) {
       const R c11 = R(vc.c11), c12 = R(vc.c12), c21 = R(vc.c21), c22 = R(vc.c22);
 #pragma unroll
       for (int k = 0; k < 6; ++k) {
         R d = Sdev.v[k] - hist[12 + k];
-        R h1 = c11 * hist[k] + c21 * d;
-        R h2 = c12 * hist[6 + k] + c22 * d;
+        R h1 = Num<R>::dot2(c11, hist[k], c21, d);
+        R h2 = Num<R>::dot2(c12, hist[6 + k], c22, d);
         hist[k] = h1;
         hist[6 + k] = h2;
         hist[12 + k] = Sdev.v[k];
@@ -568,9 +592,8 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
   if (mat == 2) {  // StVenantKirchhoff.cpp:24-41
 #pragma unroll
     for (int k = 0; k < 6; ++k) S.v[k] = R(2) * mu * E.v[k];
-    S.v[0] += lambda * trE;
-    S.v[1] += lambda * trE;
-    S.v[2] += lambda * trE;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) S.v[k] = Num<R>::add_prod(S.v[k], lambda, trE);
     return true;
   }
   const R lnJ = Num<R>::log1p_(Jm1);
@@ -583,9 +606,8 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
     Sym<R> T;
 #pragma unroll
     for (int k = 0; k < 6; ++k) T.v[k] = R(2) * mu * E.v[k];
-    T.v[0] += lambda * lnJ;
-    T.v[1] += lambda * lnJ;
-    T.v[2] += lambda * lnJ;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) T.v[k] = Num<R>::add_prod(T.v[k], lambda, lnJ);
     S = sym_mul(Ac, T, iJ2);
     return true;
   }
@@ -596,7 +618,7 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
     const R K = lambda + Num<R>::div_c(R(2) * mu, 3.0);
     const R Jm23m1 = Num<R>::expm1_(R(-2.0 / 3.0) * lnJ);
     const R Jm23 = R(1) + Jm23m1;
-    const R Ea = kappa * (R(3) * Jm23m1 + R(2) * Jm23 * trE);
+    const R Ea = kappa * Num<R>::dot2(R(3), Jm23m1, R(2) * Jm23, trE);
     R fib = R(0);
     if (Ea > R(0)) fib = R(2) * R(pp.k1) * Num<R>::exp_(R(pp.k2) * Ea * Ea) * Ea * kappa;
     const R a = Jm23 * (mu + fib);
@@ -609,12 +631,8 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
     Tdev.v[2] -= a * tr3;
     Sym<R> Sdev = sym_mul(Ac, Tdev, iJ2);
     const R pvol = R(0.5) * K * Jm1 * (Jm1 + R(2)) * iJ2;
-    S.v[0] = Sdev.v[0] + pvol * Ac.v[0];
-    S.v[1] = Sdev.v[1] + pvol * Ac.v[1];
-    S.v[2] = Sdev.v[2] + pvol * Ac.v[2];
-    S.v[3] = Sdev.v[3] + pvol * Ac.v[3];
-    S.v[4] = Sdev.v[4] + pvol * Ac.v[4];
-    S.v[5] = Sdev.v[5] + pvol * Ac.v[5];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) S.v[k] = Num<R>::add_prod(Sdev.v[k], pvol, Ac.v[k]);
     if (mat == 5 && use_hist) {
       // HGOIsotropicViscoelastic.cpp:94-159: Sdev = S - (C:S)/3 C^-1 is the
       // isochoric part above; H_j <- c1j H_j + c2j (Sdev - S0); S += H1 + H2.
@@ -622,8 +640,8 @@ __host__ __device__ inline bool pk2_stress(const PartDev &pp, const R H[3][3], R
 #pragma unroll
       for (int k = 0; k < 6; ++k) {
         R d = Sdev.v[k] - hist[12 + k];
-        R h1 = c11 * hist[k] + c21 * d;
-        R h2 = c12 * hist[6 + k] + c22 * d;
+        R h1 = Num<R>::dot2(c11, hist[k], c21, d);
+        R h2 = Num<R>::dot2(c12, hist[6 + k], c22, d);
         hist[k] = h1;
         hist[6 + k] = h2;
         hist[12 + k] = Sdev.v[k];
@@ -657,7 +675,7 @@ __host__ __device__ inline void first_piola(const PartDev &pp, const R H[3][3], 
   R C[3][3];
   adjugate(H, C);
   const R tr = H[0][0] + H[1][1] + H[2][2];
-  Jm1 = tr + ((C[0][0] + C[1][1] + C[2][2]) + (H[0][0] * C[0][0] + H[0][1] * C[1][0] + H[0][2] * C[2][0]));
+  Jm1 = tr + ((C[0][0] + C[1][1] + C[2][2]) + Num<R>::dot3(H[0][0], C[0][0], H[0][1], C[1][0], H[0][2], C[2][0]));
   const R iJ = Num<R>::rcp_(R(1) + Jm1);
   const R lnJ = Num<R>::log1p_(Jm1);
   R m, l, c4 = R(0), fa[3] = {R(0), R(0), R(0)};
@@ -677,7 +695,7 @@ __host__ __device__ inline void first_piola(const PartDev &pp, const R H[3][3], 
     l = R(0.5) * K * Jm1 * (Jm1 + R(2));
     if constexpr (MAT == 4) {
       const R kappa = R(1.0 / 3.0);
-      const R Ea = kappa * (R(3) * Jm23m1 + Jm23 * trb);
+      const R Ea = kappa * Num<R>::dot2(R(3), Jm23m1, Jm23, trb);
       R f = R(0);
       if (Ea > R(0)) f = R(2) * R(pp.k1) * Num<R>::exp_(R(pp.k2) * Ea * Ea) * Ea * kappa;
       m = Jm23 * (mu + f);
@@ -686,15 +704,15 @@ __host__ __device__ inline void first_piola(const PartDev &pp, const R H[3][3], 
       R ha[3];
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
-        ha[i] = H[i][0] * fib[0] + H[i][1] * fib[1] + H[i][2] * fib[2];
+        ha[i] = Num<R>::dot3(H[i][0], fib[0], H[i][1], fib[1], H[i][2], fib[2]);
         fa[i] = fib[i] + ha[i];
       }
       // |F a|^2 - 1 = 2 a.Ha + |Ha|^2
-      const R s4 = R(2) * (fib[0] * ha[0] + fib[1] * ha[1] + fib[2] * ha[2]) +
-                   (ha[0] * ha[0] + ha[1] * ha[1] + ha[2] * ha[2]);
+      const R s4 = R(2) * Num<R>::dot3(fib[0], ha[0], fib[1], ha[1], fib[2], ha[2]) +
+                   Num<R>::dot3(ha[0], ha[0], ha[1], ha[1], ha[2], ha[2]);
       const R I4m1 = Jm23m1 * (R(1) + s4) + s4;
-      const R I1m3 = R(3) * Jm23m1 + Jm23 * trb;
-      const R E = kappa * I1m3 + (R(1) - R(3) * kappa) * I4m1;
+      const R I1m3 = Num<R>::dot2(R(3), Jm23m1, Jm23, trb);
+      const R E = Num<R>::dot2(kappa, I1m3, R(1) - R(3) * kappa, I4m1);
       R psi = R(0);
       if (E > R(0)) psi = R(pp.k1) * E * Num<R>::exp_(R(pp.k2) * E * E);
       m = Jm23 * (mu + R(2) * psi * kappa);
@@ -704,7 +722,7 @@ __host__ __device__ inline void first_piola(const PartDev &pp, const R H[3][3], 
     l -= Num<R>::div_c(m * trb, 3.0);
   }
   const R k = (l - m) * iJ;
-  const R s = (m * Jm1 + l) * iJ + k * tr;  // m + k (1 + tr H)
+  const R s = Num<R>::dot2(Num<R>::prod_add(m, Jm1, l), iJ, k, tr);  // m + k (1 + tr H)
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -714,7 +732,7 @@ __host__ __device__ inline void first_piola(const PartDev &pp, const R H[3][3], 
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int j = 0; j < 3; ++j) P[i][j] += (c4 * fa[i]) * fib[j];
+      for (int j = 0; j < 3; ++j) P[i][j] = Num<R>::add_prod(P[i][j], c4 * fa[i], fib[j]);
   }
 }
 
@@ -1279,7 +1297,7 @@ __host__ __device__ inline void gauss_point_q(const R J0[3][3], const R Ju[3][3]
   // adj(J0): J0^-1 = A / det0 (ShapeFunction_C3D8.cpp:95-123)
   R A[3][3];
   adjugate(J0, A);
-  const R det0 = J0[0][0] * A[0][0] + J0[0][1] * A[1][0] + J0[0][2] * A[2][0];
+  const R det0 = Num<R>::dot3(J0[0][0], A[0][0], J0[0][1], A[1][0], J0[0][2], A[2][0]);
   if (!(det0 > R(0))) flags |= kFlagInverted;
   const R idet0 = Num<R>::rcp_(det0);
   // H = Ju J0^-1 = grad_X u  (F = I + H, CalculateDeformationGradient.cpp:15-25)
@@ -1288,7 +1306,7 @@ __host__ __device__ inline void gauss_point_q(const R J0[3][3], const R Ju[3][3]
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j)
-      H[i][j] = (Ju[i][0] * A[0][j] + Ju[i][1] * A[1][j] + Ju[i][2] * A[2][j]) * idet0;
+      H[i][j] = Num<R>::mul_(Num<R>::dot3(Ju[i][0], A[0][j], Ju[i][1], A[1][j], Ju[i][2], A[2][j]), idet0);
   R P[3][3], Jm1;  // P = F S (first Piola)
   if constexpr ((MAT == 1 || MAT == 4 || MAT == 8) && !SURR && !GPOUT) {
     first_piola<R, MAT>(pp, H, fib, P, Jm1);
@@ -1322,13 +1340,14 @@ __host__ __device__ inline void gauss_point_q(const R J0[3][3], const R Ju[3][3]
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j)
-        P[i][j] = sym_at(S, i, j) + H[i][0] * sym_at(S, 0, j) + H[i][1] * sym_at(S, 1, j) +
-                  H[i][2] * sym_at(S, 2, j);
+        P[i][j] = Num<R>::add_prod(Num<R>::add_prod(Num<R>::add_prod(sym_at(S, i, j), H[i][0], sym_at(S, 0, j)),
+                                                    H[i][1], sym_at(S, 1, j)),
+                                   H[i][2], sym_at(S, 2, j));
   }
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int k = 0; k < 3; ++k) Q[i][k] = P[i][0] * A[k][0] + P[i][1] * A[k][1] + P[i][2] * A[k][2];
+    for (int k = 0; k < 3; ++k) Q[i][k] = Num<R>::dot3(P[i][0], A[k][0], P[i][1], A[k][1], P[i][2], A[k][2]);
 }
 
 // One element from the unnormalised Walsh-Hadamard coefficients of its

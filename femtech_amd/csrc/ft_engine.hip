@@ -723,9 +723,9 @@ __global__ __launch_bounds__(kBlock, (elem_waves<R, MAT, WAVES>())) void k_eleme
 //   3. the 21 force coefficients in the monomial basis, shared out over the
 //      wavefronts, each summed over the points in order;
 //   4. all: the force of node w from them, corner pairs through LDS.
-// Every sum keeps element_eval's operations and order, so which kernel a
-// segment takes shows in a run by no more than the compiler's own choice of
-// fused products.  A block covers the elements of one wavefront of the
+// Every sum keeps element_eval's operations, fused or not, and their order, so
+// a run is the same to the bit whichever kernel its segments take (a mesh alone
+// takes this one, in a large batch k_element).  A block covers the elements of one wavefront of the
 // segment's tiles (63 behind a shadow lane with corner pairs, else 64), so
 // both kernels pair alike and keep the same slots.  FP64 only: the FP32 run
 // loop refines the step size of one element per tile, and a minimum over
