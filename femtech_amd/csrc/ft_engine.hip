@@ -4612,7 +4612,9 @@ int capture_chunk(ft_engine *g) {
 // later check that finds the copy complete and every instance done (end
 // time, step cap or no stable step) ends the loop, so a call asked for more
 // steps than the run has left does not keep launching kernels that exit at
-// once.  At most two check intervals of such launches are made.
+// once.  The host only polls: what it has queued by then, as far ahead of the
+// device as it gets, still runs (27^3 cube, FP64, asked for 100,000 steps: 11.6
+// ms; for its 445: 8.2 ms).
 constexpr int kDoneCheck = 128;
 
 struct DoneWatch {

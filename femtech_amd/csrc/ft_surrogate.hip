@@ -8,7 +8,7 @@
 //                layers 1-4 are stored with their input columns permuted to
 //                the accumulator layout, so one layer's output tile is the
 //                next layer's B operand as it stands).
-//   k_mlp_train  forward, loss and backward of 128 samples per block in one
+//   k_mlp_train  forward, loss and backward of 32 samples per block in one
 //                launch, leaving every layer's activations and dZ.
 //   k_mlp_grad   weight gradients per 256 samples, bias gradients.
 //   k_mlp_update gradients summed, Adam, BF16 weight copies.
@@ -285,12 +285,12 @@ __device__ inline uint64_t mix64(uint64_t z) {
 // not depend on how samples are spread over blocks.
 // A step is a chain of small products: bound by latency and by the SiLU
 // evaluations, not by the matrix cores, so the rows are split, not only the
-// samples.  A step at a batch of 1,024 / 4,096 / 65,536: 28 / 35 / 295 us (40
-// at 4,096 before k_mlp_grad's empty blocks went); 59 / 82 / 378 us with 32
-// samples and all rows per wavefront (4 to a block, weights staged in LDS,
-// SiLU' spilled); 540 us at 4,096 as 37 launches of single products and
-// elementwise passes.  At 2 wavefronts per SIMD (44 bytes of spills) instead of
-// 1, 65,536 takes 295 instead of 323 us, 4,096 the same.
+// samples.  A step at a batch of 1,024 / 4,096 / 16,384 / 65,536: 28 / 37 / 65 /
+// 303 us (all steps of a call but its first); 59 / 82 us at 1,024 / 4,096 and
+// 378 at 65,536 with 32 samples and all rows per wavefront (4 to a block,
+// weights staged in LDS, SiLU' spilled); 540 us at 4,096 as 37 launches of
+// single products and elementwise passes.  At 2 wavefronts per SIMD (44 bytes of
+// spills) instead of 1, 65,536 took 295 instead of 323 us, 4,096 the same.
 constexpr int kTrainTile = 32;      // samples per block
 constexpr int kTrainThreads = 256;  // 4 wavefronts x 32 rows of a layer
 constexpr int kGradChunk = 256;     // samples per weight-gradient block
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(kTrainThreads, 2) void k_mlp_train(TrainArgs g) {
 // an output tile each, an input tile per wavefront; layer 4: x 13), into
 // parts[z].  (Numbered through: as a grid of (14 + kDzRows) x chunks all but
 // the first chunk's bias blocks were empty; a training step at a batch of 4,096
-// / 16,384: 40 / 68 us, now 35 / 63 us.)
+// / 16,384: 40 / 68 us, then 35 / 63 us.)
 constexpr int kGradTiles = 14;
 __global__ __launch_bounds__(256) void k_mlp_grad(const __bf16 *at, const __bf16 *dzb, const float *dz, size_t ld,
                                                   float *parts, float *db) {
