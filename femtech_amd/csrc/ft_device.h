@@ -351,54 +351,62 @@ __host__ __device__ inline Sym<R> b_minus_identity(const R H[3][3]) {
 
 // 1-term Ogden (materials 6 and 7; no reference counterpart): deviatoric
 // energy (2 mu / alpha^2) sum_a (lbar_a^alpha - 1) on the isochoric principal
-// stretches, volumetric part as the reference's HGO (K/2 (J^2 - 1) in tau,
+// stretches, volumetric part as the reference's HGO (p = K/2 (J^2 - 1) in tau,
 // K = lambda + 2 mu / 3).  Kirchhoff stress tau = sum_a tau_a n_a n_a + p I
-// with tau_a = (2 mu / alpha) (lbar_a^alpha - mean_b lbar_b^alpha); the
-// stretches come from the eigenvalues of b - I (ln lbar_a = log1p(.) / 2 -
-// ln J / 3, lbar^alpha - 1 by expm1), so small strains keep full precision.
-// Returns p separately (the Prony update acts on the deviatoric part).
-template <typename R>
-__host__ __device__ inline void ogden_tau(const PartDev &pp, const Sym<R> &bm, R Jm1, Sym<R> &tau, R &p) {
-  const R mu = R(pp.mu), alpha = R(pp.alpha);
-  const R K = R(pp.lambda) + Num<R>::div_c(R(2) * mu, 3.0);
-  const R lnJ3 = Num<R>::div_c(Num<R>::log1p_(Jm1), 3.0);
-  R w[3], V[3][3];
-  sym_eig3<R, sizeof(R) == 4 ? 4 : 6>(bm, w, V);
-  R e[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) e[a] = Num<R>::expm1_(alpha * (R(0.5) * Num<R>::log1p_(w[a]) - lnJ3));
-  const R mean = Num<R>::div_c(e[0] + e[1] + e[2], 3.0);
-  const R f = R(2) * mu * Num<R>::rcp_(alpha);
-  R t[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) t[a] = f * (e[a] - mean);
-  const int I[6] = {0, 1, 2, 1, 0, 0}, J[6] = {0, 1, 2, 2, 2, 1};
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    const int i = I[k], j = J[k];
-    tau.v[k] = Num<R>::dot3(t[0] * V[i][0], V[j][0], t[1] * V[i][1], V[j][1], t[2] * V[i][2], V[j][2]);
-  }
-  p = R(0.5) * K * Jm1 * (Jm1 + R(2));
-}
+// with tau_a = (2 mu / alpha) (lbar_a^alpha - mean_b lbar_b^alpha).
+//
+// With Z = Cbar - I or bbar - I (Cbar = J^-2/3 C, bbar = J^-2/3 b) the terms
+// lbar_a^alpha - 1 are the eigenvalues of f(Z) = (I + Z)^(alpha/2) - I.  With b
+// the deviatoric stress is tau_dev = (2 mu / alpha) dev f(Z), with C (all
+// functions of C commute) S_dev = (2 mu / alpha) dev f(Z) C^-1.  f comes from
+// its power series (ogden_series) or, where that takes more terms than the
+// directions cost, from Z's principal values (ogden_principal).
 
-// Longest power series ogden_iso_series evaluates, and its tolerances (the
-// first neglected term against the leading one).
-constexpr int kOgdenTerms = 40;
+// Longest power series taken, and its tolerances (the first neglected term
+// against the leading one).
+template <typename R> __host__ __device__ constexpr int ogden_terms() { return sizeof(R) == 4 ? 24 : 40; }
 template <typename R> __host__ __device__ constexpr R ogden_tol() { return sizeof(R) == 4 ? R(3e-9) : R(1e-17); }
 
-// Isochoric PK2 stress S_dev = F^-1 dev(tau) F^-T of the 1-term Ogden law
-// without an eigen-decomposition, and C^-1.  With Z = Cbar - I (Cbar = J^-2/3
-// C) the principal terms lbar_a^alpha - 1 are the eigenvalues of f(Z) = (I +
-// Z)^(alpha/2) - I, an analytic function of Z, and S_dev = (2 mu / alpha)
-// dev(f(Z)) C^-1 (all functions of C commute).  f is summed as its binomial
-// series, each power reduced to Z^k = a I + b Z + c Z^2 by Z's characteristic
-// polynomial (three multiply-adds per power instead of a matrix product; the
-// a I terms fall out of the deviator).  No divisions, no square roots, and
-// repeated eigenvalues need no care.  Relative error against FP64 principal
-// stretches: 8e-8 to 1.1e-7 in FP32 and 6e-16 in FP64 for |Z| from 1e-5 to
-// 0.17.  Returns false, with nothing written but Ci, when |Z| is too large
-// for the series (more than kOgdenTerms terms): the caller then takes the
-// principal directions (sym_eig3).
+// The range of |Z| over which the series ends within ogden_terms terms, for p =
+// alpha / 2: any for a positive whole p, whose series is finite; else a bound
+// fitted from below to the loop's own count of terms (for alpha in -60 .. 40;
+// within 4 % of it in -20 .. 15, 14 % next to a positive whole p).  Found out by
+// running the loop to its end, larger strains paid for both ways.  110,592
+// elements, alpha -4.4, us per launch at strains of 0.01 / 0.1 / 0.2 / 0.5, before
+// and now: FP32 Ogden 25.9 / 33.4 / 41.9 / 74.1 and 23.9 / 32.2 / 41.1 / 41.6,
+// Ogden + Prony 35.0 / 42.9 / 51.0 / 83.9 and 34.5 / 42.6 / 52.4 / 51.9; FP64 Ogden
+// 62.8 / 84.3 / 170 / 171 and 50.4 / 65.1 / 102 / 103, Ogden + Prony 80.9 / 97.9 /
+// 172 / 172 and 70.3 / 91.2 / 126 / 126.  (The principal directions everywhere: 31
+// to 41, 41 to 51, 101 and 122.)
+// In FP32 for either type: with one Gauss point per lane nothing is hoisted.
+template <typename R>
+__host__ __device__ inline float ogden_range(float p) {
+  constexpr bool f32 = sizeof(R) == 4;
+  constexpr float kT = f32 ? 0.43f : 0.37f;  // (ogden_tol^(1 / ogden_terms): 0.441, 0.376)
+  if (p > 0.0f) {
+    if (p == floorf(p) && p < (float)ogden_terms<R>()) return INFINITY;
+    if (p > 20.0f) return 0.25f;
+    return fminf(Num<float>::sqrt_((f32 ? 0.245f : 0.166f) + (f32 ? 0.105f : 0.0385f) * p), 0.74f);
+  }
+  const float q = 1.0f + p;
+  return q > 0.0f ? kT * (1.0f + (f32 ? 0.15f : 0.1f) * q) : kT * Num<float>::rcp_(1.0f - (f32 ? 0.1f : 0.07f) * q);
+}
+
+// 1 / k of the FP64 series (uniform loads instead of a division per term).
+template <int N>
+struct Inverses {
+  double v[N + 1] = {};
+  __host__ __device__ constexpr Inverses() {
+    for (int k = 1; k <= N; ++k) v[k] = 1.0 / k;
+  }
+};
+
+// dev f(Z) / p by the binomial series: each power reduced to Z^k = a I + b Z + c
+// Z^2 by Z's characteristic polynomial (three multiply-adds per power instead of
+// a matrix product; the a I terms fall out of the deviator).  No divisions, no
+// square roots, and repeated eigenvalues need no care.  Q = Z^2, rho = |Z|.
+// Returns false, with nothing written, when it does not end (beyond ogden_range
+// it is not begun).
 //
 // The loop adds 7 multiply-adds per term (FP32: 5 terms at strains of 0.1 %,
 // 13 at 8 %) where the cyclic Jacobi iteration takes three rotations of about
@@ -407,10 +415,98 @@ template <typename R> __host__ __device__ constexpr R ogden_tol() { return sizeo
 // one 570 -> 450 us, 4.7 TB/s on its 2.12 GB (mostly the Prony history; a
 // plain copy of that size reaches 4.9 TB/s).
 template <typename R>
-__host__ __device__ inline bool ogden_iso_series(const PartDev &pp, const R H[3][3], R Jm1, Sym<R> &Sdev, Sym<R> &Ci) {
-  const R mu = R(pp.mu), alpha = R(pp.alpha);
+__host__ __device__ inline bool ogden_series(const Sym<R> &Z, const Sym<R> &Q, R rho, R p, Sym<R> &M) {
+  const R i1 = Z.v[0] + Z.v[1] + Z.v[2];
+  const R i2 = (Z.v[0] * Z.v[1] - Z.v[5] * Z.v[5]) + (Z.v[0] * Z.v[2] - Z.v[4] * Z.v[4]) + (Z.v[1] * Z.v[2] - Z.v[3] * Z.v[3]);
+  const R i3 = Z.v[0] * (Z.v[1] * Z.v[2] - Z.v[3] * Z.v[3]) - Z.v[5] * (Z.v[5] * Z.v[2] - Z.v[3] * Z.v[4]) +
+               Z.v[4] * (Z.v[5] * Z.v[3] - Z.v[1] * Z.v[4]);
+  // f(Z) = p Z + p (p - 1) / 2 Z^2 + ..., over the factor p: sb Z + sc Z^2
+  R ck = R(0.5) * (p - R(1)), mag = fabs(ck) * rho;  // coefficient and size of the last term added
+  R a = R(0), b = R(0), c = R(1), sb = R(1), sc = ck;
+  bool done = mag * rho <= ogden_tol<R>();
+  const float range = ogden_range<R>((float)p);
+  const int last = (float)rho <= range ? ogden_terms<R>() : 0;
+  const R shrink = range > 1.0f ? R(INFINITY) : R(0.75);
+  constexpr Inverses<ogden_terms<double>()> inv;
+#pragma unroll 1
+  for (int k = 2; k < last && !done; ++k) {
+    const R an = c * i3, bn = Num<R>::fma_(-c, i2, a), cn = Num<R>::fma_(c, i1, b);
+    a = an, b = bn, c = cn;
+    const R r = (p - R(k)) * (sizeof(R) == 4 ? Num<R>::rcp_(R(k + 1)) : R(inv.v[k + 1]));
+    ck *= r;
+    sb = Num<R>::fma_(ck, b, sb);
+    sc = Num<R>::fma_(ck, c, sc);
+    mag *= fabs(r) * rho;
+    // the terms from here on shrink at least by the factor max(|r|, 1) rho
+    done = mag * rho <= ogden_tol<R>() && rho * fmax(fabs(r), R(1)) < shrink;
+  }
+  if (!done) return false;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) M.v[k] = Num<R>::dot2(sb, Z.v[k], sc, Q.v[k]);
+  const R tr = Num<R>::div_c(M.v[0] + M.v[1] + M.v[2], 3.0);
+  M.v[0] -= tr;
+  M.v[1] -= tr;
+  M.v[2] -= tr;
+  return true;
+}
+
+// dev f(Z) from Z's principal values and directions.  (Kept out of line, its
+// call made the FP32 Ogden + Prony kernel slower than the eigen-decomposition
+// everywhere: 661 against 511 us of element kernels per step on the 2.0M
+// ellipsoid.)
+template <typename R>
+__host__ __device__ inline void ogden_principal(const Sym<R> &Z, R p, Sym<R> &M) {
+  R w[3], V[3][3];
+  sym_eig3<R, sizeof(R) == 4 ? 4 : 6>(Z, w, V);
+  R e[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) e[a] = Num<R>::expm1_(p * Num<R>::log1p_(w[a]));
+  const R mean = Num<R>::div_c(e[0] + e[1] + e[2], 3.0);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) e[a] -= mean;
   const int I[6] = {0, 1, 2, 1, 0, 0}, J[6] = {0, 1, 2, 2, 2, 1};
-  Sym<R> Z;  // C - I, then Cbar - I
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    const int i = I[k], j = J[k];
+    M.v[k] = Num<R>::dot3(e[0] * V[i][0], V[j][0], e[1] * V[i][1], V[j][1], e[2] * V[i][2], V[j][2]);
+  }
+}
+
+// M and the factor s with s M = (2 mu / alpha) dev f(Z).
+template <typename R>
+__host__ __device__ inline void ogden_dev(const PartDev &pp, const Sym<R> &Z, Sym<R> &M, R &s) {
+  const R mu = R(pp.mu), alpha = R(pp.alpha), p = R(0.5) * alpha;
+  const int I[6] = {0, 1, 2, 1, 0, 0}, J[6] = {0, 1, 2, 2, 2, 1};
+  Sym<R> Q;  // Z^2
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    const int i = I[k], j = J[k];
+    Q.v[k] = Num<R>::dot3(sym_at(Z, i, 0), sym_at(Z, j, 0), sym_at(Z, i, 1), sym_at(Z, j, 1), sym_at(Z, i, 2),
+                          sym_at(Z, j, 2));
+  }
+  const R rho = Num<R>::sqrt_(Q.v[0] + Q.v[1] + Q.v[2]);
+  s = alpha == R(0) ? R(NAN) : mu;  // 2 mu / alpha times p (no exponent: no law, as the quotient)
+  if (ogden_series(Z, Q, rho, p, M)) return;
+  ogden_principal(Z, p, M);
+  s = R(2) * mu * Num<R>::rcp_(alpha);
+}
+
+// T = C - I or b - I to J^-2/3 (I + T) - I.
+template <typename R>
+__host__ __device__ inline void isochoric(R Jm1, Sym<R> &T) {
+  const R j23 = Num<R>::expm1_(R(-2.0 / 3.0) * Num<R>::log1p_(Jm1));
+#pragma unroll
+  for (int k = 0; k < 6; ++k) T.v[k] += j23 * T.v[k];
+  T.v[0] += j23;
+  T.v[1] += j23;
+  T.v[2] += j23;
+}
+
+// Isochoric PK2 stress S_dev = F^-1 dev(tau) F^-T of the Ogden law and C^-1.
+template <typename R>
+__host__ __device__ inline void ogden_iso(const PartDev &pp, const R H[3][3], R Jm1, Sym<R> &Sdev, Sym<R> &Ci) {
+  const int I[6] = {0, 1, 2, 1, 0, 0}, J[6] = {0, 1, 2, 2, 2, 1};
+  Sym<R> Z, M;  // Z: C - I, then Cbar - I
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
     const int i = I[k], j = J[k];
@@ -426,96 +522,23 @@ __host__ __device__ inline bool ogden_iso_series(const PartDev &pp, const R H[3]
     Ci.v[4] = (Z.v[5] * Z.v[3] - Z.v[4] * c1) * iJ2;
     Ci.v[5] = (Z.v[4] * Z.v[3] - Z.v[5] * c2) * iJ2;
   }
-  const R j23 = Num<R>::expm1_(R(-2.0 / 3.0) * Num<R>::log1p_(Jm1));
-#pragma unroll
-  for (int k = 0; k < 6; ++k) Z.v[k] += j23 * Z.v[k];
-  Z.v[0] += j23;
-  Z.v[1] += j23;
-  Z.v[2] += j23;
-  Sym<R> Q;  // Z^2
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    const int i = I[k], j = J[k];
-    Q.v[k] = Num<R>::dot3(sym_at(Z, i, 0), sym_at(Z, j, 0), sym_at(Z, i, 1), sym_at(Z, j, 1), sym_at(Z, i, 2),
-                          sym_at(Z, j, 2));
-  }
-  const R i1 = Z.v[0] + Z.v[1] + Z.v[2];
-  const R i2 = (Z.v[0] * Z.v[1] - Z.v[5] * Z.v[5]) + (Z.v[0] * Z.v[2] - Z.v[4] * Z.v[4]) + (Z.v[1] * Z.v[2] - Z.v[3] * Z.v[3]);
-  const R i3 = Z.v[0] * (Z.v[1] * Z.v[2] - Z.v[3] * Z.v[3]) - Z.v[5] * (Z.v[5] * Z.v[2] - Z.v[3] * Z.v[4]) +
-               Z.v[4] * (Z.v[5] * Z.v[3] - Z.v[1] * Z.v[4]);
-  const R rho2 = Q.v[0] + Q.v[1] + Q.v[2];  // |Z|^2
-  const R rho = Num<R>::sqrt_(rho2);
-  // f(Z) = p Z + p (p - 1) / 2 Z^2 + ..., p = alpha / 2, over the factor p:
-  // sb Z + sc Z^2
-  const R p = R(0.5) * alpha;
-  R ck = R(0.5) * (p - R(1)), mag = fabs(ck) * rho;  // coefficient and size of the last term added
-  R a = R(0), b = R(0), c = R(1), sb = R(1), sc = ck;
-  bool done = mag * rho <= ogden_tol<R>();
-#pragma unroll 1
-  for (int k = 2; k < kOgdenTerms && !done; ++k) {
-    const R an = c * i3, bn = Num<R>::fma_(-c, i2, a), cn = Num<R>::fma_(c, i1, b);
-    a = an, b = bn, c = cn;
-    const R r = (p - R(k)) * (sizeof(R) == 4 ? Num<R>::rcp_(R(k + 1)) : R(1) / R(k + 1));
-    ck *= r;
-    sb = Num<R>::fma_(ck, b, sb);
-    sc = Num<R>::fma_(ck, c, sc);
-    mag *= fabs(r) * rho;
-    // the terms from here on shrink at least by the factor max(|r|, 1) rho
-    done = mag * rho <= ogden_tol<R>() && rho * fmax(fabs(r), R(1)) < R(0.75);
-  }
-  if (!done) return false;
-  Sym<R> M;
-#pragma unroll
-  for (int k = 0; k < 6; ++k) M.v[k] = Num<R>::dot2(sb, Z.v[k], sc, Q.v[k]);
-  const R tr = Num<R>::div_c(M.v[0] + M.v[1] + M.v[2], 3.0);
-  M.v[0] -= tr;
-  M.v[1] -= tr;
-  M.v[2] -= tr;
-  // 2 mu / alpha times the factor p (no exponent: no law, as the quotient)
-  Sdev = sym_mul(Ci, M, alpha == R(0) ? R(NAN) : mu);
-  return true;
+  isochoric(Jm1, Z);
+  R s;
+  ogden_dev(pp, Z, M, s);
+  Sdev = sym_mul(Ci, M, s);
 }
 
-// The same from the principal stretches (ogden_tau), for strains beyond the
-// series.  (Kept out of line, its call made the FP32 Ogden + Prony kernel
-// slower than the eigen-decomposition everywhere: 661 against 511 us of
-// element kernels per step on the 2.0M ellipsoid.)
+// Kirchhoff stress of the Ogden law (material 6).
 template <typename R>
-__host__ __device__ inline void ogden_iso_principal(const PartDev &pp, const R H[3][3], R Jm1, Sym<R> &Sdev,
-                                                    Sym<R> &Ci) {
-  Sym<R> td;
-  R p;
-  ogden_tau(pp, b_minus_identity(H), Jm1, td, p);
-  R F[3][3], Fi[3][3];
+__host__ __device__ inline void ogden_tau(const PartDev &pp, const R H[3][3], R Jm1, Sym<R> &tau) {
+  const R K = R(pp.lambda) + Num<R>::div_c(R(2) * R(pp.mu), 3.0);
+  const R p = Num<R>::mul_(R(0.5) * K * Jm1, Jm1 + R(2));
+  Sym<R> Z = b_minus_identity(H), M;
+  isochoric(Jm1, Z);
+  R s;
+  ogden_dev(pp, Z, M, s);
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) F[i][j] = H[i][j] + (i == j ? R(1) : R(0));
-  adjugate(F, Fi);
-  const R iJ = Num<R>::rcp_(R(1) + Jm1);
-  const int I[6] = {0, 1, 2, 1, 0, 0}, J[6] = {0, 1, 2, 2, 2, 1};
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) Fi[i][j] *= iJ;
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    const int i = I[k], j = J[k];
-    R sd = R(0), ci = R(0);
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      ci += Fi[i][a] * Fi[j][a];
-#pragma unroll
-      for (int b = 0; b < 3; ++b) sd += Fi[i][a] * sym_at(td, a, b) * Fi[j][b];
-    }
-    Sdev.v[k] = sd;
-    Ci.v[k] = ci;
-  }
-}
-
-template <typename R>
-__host__ __device__ inline void ogden_iso(const PartDev &pp, const R H[3][3], R Jm1, Sym<R> &Sdev, Sym<R> &Ci) {
-  if (!ogden_iso_series(pp, H, Jm1, Sdev, Ci)) ogden_iso_principal(pp, H, Jm1, Sdev, Ci);
+  for (int k = 0; k < 6; ++k) tau.v[k] = k < 3 ? Num<R>::add_prod(p, s, M.v[k]) : s * M.v[k];
 }
 
 struct ViscoCoef { double c11, c12, c21, c22; };
@@ -1308,7 +1331,29 @@ __host__ __device__ inline void gauss_point_q(const R J0[3][3], const R Ju[3][3]
     for (int j = 0; j < 3; ++j)
       H[i][j] = Num<R>::mul_(Num<R>::dot3(Ju[i][0], A[0][j], Ju[i][1], A[1][j], Ju[i][2], A[2][j]), idet0);
   R P[3][3], Jm1;  // P = F S (first Piola)
-  if constexpr ((MAT == 1 || MAT == 4 || MAT == 8) && !SURR && !GPOUT) {
+  if constexpr (MAT == 6 && !SURR && !GPOUT) {
+    // Spatial form: P J0^-T = tau F^-T J0^-T = tau Jx^-T with the deformed
+    // Jacobian Jx = F J0 = J0 + Ju, so Q = tau adj(Jx)^T / J.  The law's own
+    // stress is spatial: no C^-1, no pull-back and no F S.
+    Jm1 = det_ip1_m1(H);
+    if (!(Jm1 > R(-1))) flags |= kFlagInverted;
+    Sym<R> tau;
+    ogden_tau(pp, H, Jm1, tau);
+    const R iJ = Num<R>::rcp_(R(1) + Jm1);
+    R X[3][3], B[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) X[i][j] = J0[i][j] + Ju[i][j];
+    adjugate(X, B);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const R t0 = sym_at(tau, i, 0) * iJ, t1 = sym_at(tau, i, 1) * iJ, t2 = sym_at(tau, i, 2) * iJ;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) Q[i][k] = Num<R>::dot3(t0, B[k][0], t1, B[k][1], t2, B[k][2]);
+    }
+    return;
+  } else if constexpr ((MAT == 1 || MAT == 4 || MAT == 8) && !SURR && !GPOUT) {
     first_piola<R, MAT>(pp, H, fib, P, Jm1);
     if (!(Jm1 > R(-1))) flags |= kFlagInverted;
   } else {

@@ -3088,11 +3088,11 @@ int force_segment(ft_engine *g, const ft_engine::Seg &sg, int waves, bool in_loo
 // kWaveLaunch us.  Measured on jittered blocks of one law, us per launch of
 // k_element / k_element_waves at 1,000, 8,000, 32,768 and 97,336 elements:
 // neo-Hookean 16.8 / 11.0, 17.3 / 11.6, 18.7 / 21.3, 28.8 / 39.8; HGO + Prony
-// 27.8 / 13.4, 28.9 / 15.5, 31.4 / 29.4, 58.6 / 70.9; Ogden + Prony 83.3 /
-// 31.4, 95.0 / 29.1, 55.9 / 37.2, 86.6 / 83.2, and 88.4 / 93.5 at 103,823, 88.3 /
-// 104.5 at 115,248; Ogden 81.0 / 81.1 at 89,100; anisotropic HGO 23.5 / 11.9,
-// 23.7 / 12.1, 22.4 / 22.7, 42.0 / 44.3.  The launch shapes of
-// ft_set_segment_shape and ft_autotune apply to k_element only.
+// 27.8 / 13.4, 28.9 / 15.5, 31.4 / 29.4, 58.6 / 70.9; anisotropic HGO 23.5 / 11.9,
+// 23.7 / 12.1, 22.4 / 22.7, 42.0 / 44.3; Ogden (alpha -4.4) at 32,768, 89,100 and
+// 129,792 elements 67.8 / 33.1, 66.4 / 50.8, 86.7 / 68.5; Ogden + Prony at 32,768,
+// 97,336, 108,288 and 120,050: 74.1 / 40.9, 89.7 / 90.5, 96.1 / 100.1, 97.6 / 109.3.
+// The launch shapes of ft_set_segment_shape and ft_autotune apply to k_element only.
 struct WaveCost {
   double alone;  // us
   int even;      // elements
@@ -3102,7 +3102,7 @@ WaveCost wave_cost(int mat) {
   switch (mat) {
     case 4: return {19, 65000};
     case 5: return {26, 60000};
-    case 6: return {40, 120000};
+    case 6: return {40, 176000};
     case 7: return {60, 118000};
     case 8: return {21, 65000};
     default: return {15, 80000};
