@@ -3081,46 +3081,65 @@ int force_segment(ft_engine *g, const ft_engine::Seg &sg, int waves, bool in_loo
   return fail(FT_ERR_MATERIAL, "Unknown material type %d", sg.mat);
 }
 
-// When k_element_waves takes a run of consecutive FP64 material segments: each
-// segment's own k_element launch costs `alone` us however small it is; as
-// part of a k_element_waves launch it costs time in proportion to its
-// elements, the same at `even` of them; and that launch itself costs
-// kWaveLaunch us.  Measured on jittered blocks of one law, us per launch of
+// When k_element_waves takes FP64 material segments.  A segment's own k_element
+// launch costs `alone` us however small it is; a k_element_waves launch costs
+// kWaveLaunch us and time in proportion to its elements, for one law the same as
+// k_element at `even` of them, for several laws (the kernel then has the registers
+// of the dearest) at `shared`: net of the fifth by which k_element's time grows up
+// to 60,000 elements.  Measured on jittered blocks of one law, us per launch of
 // k_element / k_element_waves at 1,000, 8,000, 32,768 and 97,336 elements:
 // neo-Hookean 16.8 / 11.0, 17.3 / 11.6, 18.7 / 21.3, 28.8 / 39.8; HGO + Prony
 // 27.8 / 13.4, 28.9 / 15.5, 31.4 / 29.4, 58.6 / 70.9; anisotropic HGO 23.5 / 11.9,
 // 23.7 / 12.1, 22.4 / 22.7, 42.0 / 44.3; Ogden (alpha -4.4) at 32,768, 89,100 and
 // 129,792 elements 67.8 / 33.1, 66.4 / 50.8, 86.7 / 68.5; Ogden + Prony at 32,768,
 // 97,336, 108,288 and 120,050: 74.1 / 40.9, 89.7 / 90.5, 96.1 / 100.1, 97.6 / 109.3.
+// Several laws, us per step of a k_element launch each / of one k_element_waves for
+// all, equal parts of 2,000, 16,000, 24,000, 32,000, 44,000 and 58,000 elements each:
+// laws 1, 2 31.7 / 11.4, 33.4 / 27.4, 35.2 / 35.2, 37.3 / 37.0, 40.4 / 51.0, 43.8 /
+// 65.5; 1, 2, 3 47.5 / 11.6, 51.3 / 35.3, 54.0 / 43.4, 58.3 / 57.2, 61.0 / 71.8, 62.9 /
+// 88.9; 1 to 5 96.7 / 14.3, 105 / 55.8, 108 / 74.2, 109 / 90.8, 114 / 120, 120 / 157;
+// 5, 7 71.4 / 16.7, 74.3 / 38.8, 75.4 / 51.5, 75.9 / 55.8, 77.5 / 75.8, 82.9 / 97.9;
+// 3, 7, 8 79.3 / 16.7, 81.9 / 41.7, 84.3 / 52.1, 86.8 / 69.4, 89.8 / 88.2, 94.1 / 109;
+// 1 to 8 195 / 20.1, 207 / 85.2, 206 / 117, 208 / 148, 214 / 197.  A k_element_waves
+// launch for each: 1, 2 at 24,000 30.4; 5, 7 at 32,000 61.9; 6, 7 at 100,000 130
+// against 152 for the one.  The Ogden rows cost k_element less the smaller the
+// strains: Ogden + Prony below a percent takes it 53 at 58,000, k_element_waves 60,
+// and from 66,000 on 85 against 70.
 // The launch shapes of ft_set_segment_shape and ft_autotune apply to k_element only.
 struct WaveCost {
-  double alone;  // us
-  int even;      // elements
+  double alone;      // us
+  int even, shared;  // elements
 };
 constexpr double kWaveLaunch = 10.5;  // us
 WaveCost wave_cost(int mat) {
   switch (mat) {
-    case 4: return {19, 65000};
-    case 5: return {26, 60000};
-    case 6: return {40, 176000};
-    case 7: return {60, 118000};
-    case 8: return {21, 65000};
-    default: return {15, 80000};
+    case 4: return {19, 65000, 38500};
+    case 5: return {26, 60000, 55000};
+    case 6: return {40, 176000, 110000};
+    case 7: return {60, 118000, 100000};
+    case 8: return {21, 65000, 40000};
+    default: return {17, 80000, 37500};
   }
 }
 
-// End of the run of segments from s on that k_element_waves takes (s: none).
+// End of the run of segments from s on that k_element_waves takes (s: none): the
+// longest run whose shared launch gains more than its segments' own would, else
+// the segment by itself.
 size_t wave_run(const ft_engine *g, size_t s) {
   if (g->precision == FT_FP32) return s;
-  double gain = -kWaveLaunch;
-  size_t s1 = s;
-  for (; s1 < g->segs.size(); ++s1) {
+  size_t best = s;
+  double together = -kWaveLaunch, apart = 0.0;  // us gained over k_element
+  for (size_t s1 = s; s1 < g->segs.size(); ++s1) {
     const WaveCost c = wave_cost(g->segs[s1].mat);
     const int ne = g->segs[s1].end - g->segs[s1].begin;
-    if (ne >= c.even) break;
-    gain += c.alone * (1.0 - (double)ne / c.even);
+    const double own = c.alone * (1.0 - (double)ne / c.even) - kWaveLaunch;
+    if (s1 == s && own > 0.0) best = s + 1;
+    if (ne >= c.shared) break;
+    together += c.alone * (1.0 - (double)ne / c.shared);
+    apart += std::max(0.0, own);
+    if (s1 > s && together > apart) best = s1 + 1;
   }
-  return gain > 0.0 ? s1 : s;
+  return best;
 }
 
 // k_element_waves over segments [s0, s1), contiguous in the internal order.
